@@ -51,7 +51,7 @@ struct AdjArgs {
   double rk_b_next;         // mode 1: b of the next reverse stage
   unsigned *err;
   PhysParams ph;
-  BCTable bc;
+  const BCTable *bc;
 };
 
 template <int N>
@@ -631,9 +631,9 @@ __global__ void __launch_bounds__((64 * AdjGroup<N, EQN>::W), (AdjWaves<N, EQN>:
         const double z = a.I1D[3 * Ng * Nfp + g], s = 0.5 * (1.0 + z);
         const double xg = vk[2 * va] + s * (vk[2 * vb] - vk[2 * va]);
         const double yg = vk[2 * va + 1] + s * (vk[2 * vb + 1] - vk[2 * va + 1]);
-        boundary_state<EQN>(a.bc, -code - 1, a.t, xg, yg, nx, ny, qM, qP);
+        boundary_state<EQN>(*a.bc, -code - 1, a.t, xg, yg, nx, ny, qM, qP);
         num_flux_vjp<EQN, FLUX>(a.ph, nx, ny, qM, qP, nb, qMb, qPb);
-        boundary_vjp<EQN>(a.bc, -code - 1, nx, ny, qPb, qMb);
+        boundary_vjp<EQN>(*a.bc, -code - 1, nx, ny, qPb, qMb);
       }
     }
 #pragma unroll

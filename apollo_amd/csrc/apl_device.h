@@ -115,7 +115,9 @@ struct RhsArgs {
   double *speed_part;      // [nbatch] max LF speed per batch, or null
   unsigned *err;           // error flags
   PhysParams ph;
-  BCTable bc;
+  const BCTable *bc;       // device copy: kernel arguments sit in host memory, which
+                           // a lane's own index would read across the bus
+  int vortex;              // some boundary is the isentropic vortex
 };
 
 // ---------------------------------------------------------------------------
@@ -203,6 +205,23 @@ __device__ __forceinline__ float recip(float x) {
   return fmaf(r, e, r);
 }
 
+// sqrt(x) for x >= 0 by Goldschmidt's iteration from the hardware reciprocal
+// square root estimate: one coupled step and a residual correction, within an
+// ulp, in 9 instructions instead of the 17 of the IEEE-exact sequence (which
+// scales for subnormals and selects for 0 and infinity).  Arguments below
+// 2^-1000, 0 among them, return about 2^-500: next to nothing in a wave
+// speed.  A negative or NaN argument does the same (such a state raises its
+// own flag).
+__device__ __forceinline__ double root(double x) {
+  x = fmax(x, 0x1p-1000);
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double e = fma(-h, g, 0.5);
+  g = fma(g, e, g);
+  h = fma(h, e, h);
+  return fma(fma(-g, g, x), h, g);
+}
+
 // Physical fluxes F (x) and G (y) of WxEulerEqn::flux (wxeulereqn.cc:806-871)
 // and WxPHMaxwellEqn::flux (wxphmaxwelleqn.cc:447-498).  EULER4 is EULER5
 // with rho w == 0 and that component dropped; TM3 is the (Ez, Bx, By) subset
@@ -246,15 +265,91 @@ __device__ __forceinline__ unsigned phys_flux(const PhysParams &P, const S *q, S
   return ef;
 }
 
-// Euler flux of one trace and its LF wave speed |u| + c
+// Density (floored), its reciprocal, velocities and pressure of an Euler
+// state, as phys_flux forms them, and its flags.
+template <int EQN>
+__device__ __forceinline__ unsigned euler_prim(const PhysParams &P, const double *q, double &rho,
+                                               double &ir, double &u, double &v, double &w, double &p) {
+  constexpr bool W = (EQN == APL_EQN_EULER5);
+  rho = q[0];
+  const bool bad_rho = P.min_dens == 0.0 && !(rho > 0.0);
+  if (rho < P.min_dens) rho = P.min_dens;
+  ir = recip(rho);
+  u = q[1] * ir;
+  v = q[2] * ir;
+  w = W ? q[3] * ir : 0.0;
+  p = (P.gamma - 1.0) * (q[W ? 4 : 3] - 0.5 * rho * (u * u + v * v + w * w));
+  const bool low = !(p > 0.0);
+  if (low && P.min_pres != 0.0) p = P.min_pres;
+  return (bad_rho ? EF_DENSITY : 0u) | (low && P.min_pres == 0.0 ? EF_PRESSURE : 0u);
+}
+
+// Contravariant fluxes pr = jrx F + jry G, ps = jsx F + jsy G of a cubature
+// point (FP64).  Euler: from the contravariant velocity of each direction,
+// 16 instructions after the primitives where F, G and their combination
+// take 26.
+template <int EQN>
+__device__ __forceinline__ unsigned point_flux(const PhysParams &P, double jrx, double jry, double jsx,
+                                               double jsy, const double *q, double *pr, double *ps) {
+  constexpr int M = Vars<EQN>::M;
+  if constexpr (EQN == APL_EQN_EULER5 || EQN == APL_EQN_EULER4) {
+    constexpr int IE = M - 1;
+    double rho, ir, u, v, w, p;
+    const unsigned ef = euler_prim<EQN>(P, q, rho, ir, u, v, w, p);
+    const double ur = jrx * u + jry * v, us = jsx * u + jsy * v, h = q[IE] + p;
+    pr[0] = rho * ur;
+    ps[0] = rho * us;
+    pr[1] = pr[0] * u + jrx * p;
+    ps[1] = ps[0] * u + jsx * p;
+    pr[2] = pr[0] * v + jry * p;
+    ps[2] = ps[0] * v + jsy * p;
+    if constexpr (M == 5) {
+      pr[3] = pr[0] * w;
+      ps[3] = ps[0] * w;
+    }
+    pr[IE] = h * ur;
+    ps[IE] = h * us;
+    return ef;
+  } else {
+    double F[M], G[M];
+    const unsigned ef = phys_flux<EQN, double>(P, q, F, G);
+#pragma unroll
+    for (int v = 0; v < M; ++v) {
+      pr[v] = jrx * F[v] + jry * G[v];
+      ps[v] = jsx * F[v] + jsy * G[v];
+    }
+    return ef;
+  }
+}
+
+// Normal flux f = nx F + ny G of one Euler trace and its LF wave speed |u| + c
 // (wxeulereqn.cc:806-871, 1106-1110) from one reciprocal of the density and
-// one pressure; the density and pressure floors act as in phys_flux.
-// Square roots of the LF wave speed: IEEE for FP64; the hardware's for FP32
-// (within an ulp), in the FP32 face flux of the FP32 and split-BF16x3 kernels.
-__device__ __forceinline__ double speed_sqrt(double x) { return sqrt(x); }
+// one pressure; the density and pressure floors act as in phys_flux.  The
+// normal velocity is formed first, so that only one flux is built.
+template <int EQN>
+__device__ __forceinline__ unsigned euler_normal_flux(const PhysParams &P, double nx, double ny,
+                                                      const double *q, double *f, double *speed) {
+  constexpr bool W = (EQN == APL_EQN_EULER5);
+  constexpr int IE = W ? 4 : 3;
+  double rho, ir, u, v, w, p;
+  const unsigned ef = euler_prim<EQN>(P, q, rho, ir, u, v, w, p);
+  const double k2 = u * u + v * v + w * w;
+  const double un = nx * u + ny * v, mn = rho * un;
+  f[0] = mn;
+  f[1] = mn * u + nx * p;
+  f[2] = mn * v + ny * p;
+  if constexpr (W) f[3] = mn * w;
+  f[IE] = (q[IE] + p) * un;
+  *speed = root(k2) + root(P.gamma * p * ir);
+  return ef;
+}
+
+// The square root of the FP32 wave speed: the hardware's, within an ulp, in
+// the FP32 face flux of the FP32 and split-BF16x3 kernels.
 __device__ __forceinline__ float speed_sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 
-template <int EQN, typename S = double>
+// FP32 fluxes F, G and wave speed of one trace, as euler_normal_flux.
+template <int EQN, typename S>
 __device__ __forceinline__ unsigned euler_flux_speed(const PhysParams &P, const S *q, S *F, S *G,
                                                      S *speed) {
   constexpr bool W = (EQN == APL_EQN_EULER5);
@@ -329,25 +424,26 @@ __device__ __forceinline__ unsigned euler_riemann_flux(const PhysParams &P, doub
   unsigned ef = phys_flux<EQN, double>(P, qM, FM, GM);
   ef |= phys_flux<EQN, double>(P, qP, FP, GP);
   // rotated primitives: rho, u (normal), v, w, p
-  const double iM = 1.0 / qM[0], iP = 1.0 / qP[0];
+  const double iM = recip(qM[0]), iP = recip(qP[0]);
   const double uM = qM[1] * iM, vM = qM[2] * iM, wM = W ? qM[3] * iM : 0.0;
   const double uP = qP[1] * iP, vP = qP[2] * iP, wP = W ? qP[3] * iP : 0.0;
   const double mwM = W ? qM[3] : 0.0, mwP = W ? qP[3] : 0.0;
   const double pM = (g - 1.) * (qM[IE] - 0.5 * (qM[1] * qM[1] + qM[2] * qM[2] + mwM * mwM) * iM);
   const double pP = (g - 1.) * (qP[IE] - 0.5 * (qP[1] * qP[1] + qP[2] * qP[2] + mwP * mwP) * iP);
-  const double cM = sqrt(g * pM * iM), cP = sqrt(g * pP * iP);
+  const double cM = root(g * pM * iM), cP = root(g * pP * iP);
   // Roe averages
   const double HM = (qM[IE] + pM) * iM, HP = (qP[IE] + pP) * iP;
-  const double rM = sqrt(qM[0]), rP = sqrt(qP[0]), irs = 1.0 / (rM + rP);
+  const double rM = root(qM[0]), rP = root(qP[0]), irs = recip(rM + rP);
   const double u = (rM * uM + rP * uP) * irs, v = (rM * vM + rP * vP) * irs;
   const double w = (rM * wM + rP * wP) * irs, H = (rM * HM + rP * HP) * irs;
-  const double c2 = (g - 1.) * (H - 0.5 * (u * u + v * v + w * w)), c = sqrt(c2);
+  const double c2 = (g - 1.) * (H - 0.5 * (u * u + v * v + w * w)), c = root(c2);
   double fx[M];
   if constexpr (FLUX == APL_FLUX_HLL) {
     const double SL = fmin(uM - cM, u - c), SR = fmax(uP + cP, u + c);
-    const double t1 = (fmin(SR, 0.0) - fmin(0.0, SL)) / (SR - SL);
+    const double is = recip(SR - SL);
+    const double t1 = (fmin(SR, 0.0) - fmin(0.0, SL)) * is;
     const double t2 = 1. - t1;
-    const double t3 = (SR * fabs(SL) - SL * fabs(SR)) / (2. * (SR - SL));
+    const double t3 = 0.5 * (SR * fabs(SL) - SL * fabs(SR)) * is;
 #pragma unroll
     for (int k = 0; k < M; ++k) fx[k] = t1 * FP[k] + t2 * FM[k] - t3 * (qP[k] - qM[k]);
     fs[1] = nx * fx[1] - ny * fx[2];
@@ -375,8 +471,8 @@ __device__ __forceinline__ unsigned euler_riemann_flux(const PhysParams &P, doub
   fs[0] = fx[0];
   if constexpr (W) fs[3] = 0.0;
   fs[IE] = fx[IE];
-  const double lM = sqrt(uM * uM + vM * vM + wM * wM) + cM;
-  const double lP = sqrt(uP * uP + vP * vP + wP * wP) + cP;
+  const double lM = root(uM * uM + vM * vM + wM * wM) + cM;
+  const double lP = root(uP * uP + vP * vP + wP * wP) + cP;
   *lam = lM > lP ? lM : lP;
   return ef;
 }
@@ -408,22 +504,22 @@ __device__ __forceinline__ unsigned num_flux(const PhysParams &P, double nx, dou
     rP[2] = -ny * qP[1] + nx * qP[2];
     return num_flux<EQN, APL_FLUX_LF>(P, nx, ny, rM, rP, fs, lam);
   }
-  double FM[M], GM[M], FP[M], GP[M];
-  unsigned ef = 0;
-  double l;
   if constexpr (EQN == APL_EQN_EULER5 || EQN == APL_EQN_EULER4) {
-    // flux and |u| + c of each trace from one reciprocal and one pressure
-    double cM, cP;
-    ef |= euler_flux_speed<EQN>(P, qM, FM, GM, &cM);
-    ef |= euler_flux_speed<EQN>(P, qP, FP, GP, &cP);
-    l = cM > cP ? cM : cP;
-  } else {
-    ef |= phys_flux<EQN, double>(P, qM, FM, GM);
-    ef |= phys_flux<EQN, double>(P, qP, FP, GP);
-    const double a = P.chi * P.c0, b = P.gph * P.c0;
-    const double m1 = a > b ? a : b;
-    l = m1 > P.c0 ? m1 : P.c0;
+    double fM[M], fP[M], cM, cP;
+    unsigned ef = euler_normal_flux<EQN>(P, nx, ny, qM, fM, &cM);
+    ef |= euler_normal_flux<EQN>(P, nx, ny, qP, fP, &cP);
+    const double l = fmax(cM, cP);   // root() gives no NaN
+#pragma unroll
+    for (int c = 0; c < M; ++c) fs[c] = 0.5 * (fM[c] + fP[c] + l * (qM[c] - qP[c]));
+    *lam = l;
+    return ef;
   }
+  double FM[M], GM[M], FP[M], GP[M];
+  unsigned ef = phys_flux<EQN, double>(P, qM, FM, GM);
+  ef |= phys_flux<EQN, double>(P, qP, FP, GP);
+  const double a = P.chi * P.c0, b = P.gph * P.c0;
+  const double m1 = a > b ? a : b;
+  const double l = m1 > P.c0 ? m1 : P.c0;
 #pragma unroll
   for (int c = 0; c < M; ++c)
     fs[c] = 0.5 * (nx * (FM[c] + FP[c]) + ny * (GM[c] + GP[c]) + l * (qM[c] - qP[c]));
@@ -465,16 +561,25 @@ __device__ __forceinline__ void store_euler5(const double *q5, double *q) {
   }
 }
 
+// A boundary state that depends on nothing but its parameters (inflow,
+// Dirichlet), as the kernels see it: BCTable.p holds the conserved state
+// (rho, rho u, rho v, rho w, E), formed once per call on the host.
+constexpr int BC_FIXED = 64;
+
 // Euler exterior states on the 5-variable state: isentropic vortex
-// (wxisentropicvortexbc.cc:20-43), wall (wxeulerwallbc.cc:18-25), inflow
-// (wxeulerinflowbc.cc:21-36), Dirichlet (wxeulerdirichletbc.cc:22-30); any
-// other kind copies (zero gradient, wxeulerzerogradientbc.cc:18-25).
+// (wxisentropicvortexbc.cc:20-43), wall (wxeulerwallbc.cc:18-25), fixed
+// states (inflow, wxeulerinflowbc.cc:21-36; Dirichlet,
+// wxeulerdirichletbc.cc:22-30); any other kind copies (zero gradient,
+// wxeulerzerogradientbc.cc:18-25).  VTX = false leaves the vortex out, for
+// kernels that no handle with that boundary reaches: its exp and pow take
+// most of a kernel's registers.
+template <bool VTX = true>
 __device__ __forceinline__ void euler_bc5(int kind, const double *p, double t, double x, double y,
                                           double nx, double ny, const double *q, double *o) {
 #pragma unroll
   for (int c = 0; c < 5; ++c) o[c] = q[c];
-  const double pi = 3.141592653589793;
-  if (kind == APL_BC_ISENTROPIC_VORTEX) {
+  if (VTX && kind == APL_BC_ISENTROPIC_VORTEX) {
+    const double pi = 3.141592653589793;
     const double uo = p[0], vo = p[1], xo = p[2], yo = p[3], gamma = p[4], beta = p[5];
     const double xmut = x - uo * t, ymvt = y - vo * t;
     const double r = sqrt((xmut - xo) * (xmut - xo) + (ymvt - yo) * (ymvt - yo));
@@ -494,30 +599,16 @@ __device__ __forceinline__ void euler_bc5(int kind, const double *p, double t, d
     o[1] = q[1] - 2. * qn * nx;
     o[2] = q[2] - 2. * qn * ny;
     o[3] = 0.0;
-  } else if (kind == APL_BC_EULER_INFLOW) {
-    const double mach = p[0], angle = p[1], gamma = p[2], pres = p[3], rho = p[4];
-    const double sound = sqrt(gamma * pres / rho);
-    const double u = mach * sound * cos(angle * pi / 180.);
-    const double v = mach * sound * sin(angle * pi / 180.);
-    o[0] = rho;
-    o[1] = rho * u;
-    o[2] = rho * v;
-    o[3] = 0.0;
-    o[4] = pres / (gamma - 1) + 0.5 * rho * (u * u + v * v);
-  } else if (kind == APL_BC_EULER_DIRICHLET) {
-    const double rho = p[0], u = p[1], v = p[2], w = p[3], gamma = p[4], pres = p[5];
-    o[0] = rho;
-    o[1] = rho * u;
-    o[2] = rho * v;
-    o[3] = rho * w;
-    o[4] = pres / (gamma - 1) + 0.5 * rho * (u * u + v * v + w * w);
+  } else if (kind == BC_FIXED) {
+#pragma unroll
+    for (int c = 0; c < 5; ++c) o[c] = p[c];
   }
 }
 
 // Exterior state at a boundary Gauss point (wxgridbc.cc:21-26 and
 // wxisentropicvortexbc.cc:20-43, wxmaxwelltranversemagneticbc.cc:13-25,
 // wxphmaxwellconductingwallbc.cc:12-41).
-template <int EQN>
+template <int EQN, bool VTX = true>
 __device__ __forceinline__ void boundary_state(const BCTable &B, int idx, double t, double x,
                                                double y, double nx, double ny, const double *qM,
                                                double *qP) {
@@ -530,7 +621,7 @@ __device__ __forceinline__ void boundary_state(const BCTable &B, int idx, double
     if (kind != APL_BC_COPY && kind != APL_BC_NONE) {
       double q5[5], o5[5];
       load_euler5<EQN>(qM, q5);
-      euler_bc5(kind, p, t, x, y, nx, ny, q5, o5);
+      euler_bc5<VTX>(kind, p, t, x, y, nx, ny, q5, o5);
       store_euler5<EQN>(o5, qP);
     }
   } else if constexpr (EQN == APL_EQN_PHMAXWELL8) {
@@ -872,7 +963,7 @@ __device__ __forceinline__ void face_flux_cub(const RhsArgs &a, int ks, S *fsT, 
         double dM[M], dP[M];
 #pragma unroll
         for (int v = 0; v < M; ++v) dM[v] = qM[v];
-        boundary_state<EQN>(a.bc, -code - 1, F.tnow, xg, yg, nx, ny, dM, dP);
+        boundary_state<EQN>(*a.bc, -code - 1, F.tnow, xg, yg, nx, ny, dM, dP);
 #pragma unroll
         for (int v = 0; v < M; ++v) qP[v] = float(dP[v]);
       }
@@ -928,7 +1019,7 @@ __device__ __forceinline__ void face_flux_cub(const RhsArgs &a, int ks, S *fsT, 
       const double s = 0.5 * (1.0 + z);
       const double xg = vk[2 * va] + s * (vk[2 * vb] - vk[2 * va]);
       const double yg = vk[2 * va + 1] + s * (vk[2 * vb + 1] - vk[2 * va + 1]);
-      boundary_state<EQN>(a.bc, -code - 1, F.tnow, xg, yg, nx, ny, qM, qP);
+      boundary_state<EQN>(*a.bc, -code - 1, F.tnow, xg, yg, nx, ny, qM, qP);
     }
     double lam;
     F.ef |= num_flux<EQN, FLUX>(a.ph, nx, ny, qM, qP, fs, &lam);
@@ -1465,7 +1556,7 @@ __global__ void __launch_bounds__((64 * LinGroup<N, EQN, T>::W), (LinWaves<N, EQ
       if constexpr (!PRE) gather_face_node<Np, Nfp, M>(qg, kf, code0, code1, code2, fnb[ks], qp);
 #pragma unroll
       for (int v = 0; v < M; ++v) qM[v] = double(XT[(fown[ks] * M + v) * XS + el]);
-      if (code < 0) boundary_state<EQN>(a.bc, -code - 1, 0.0, 0.0, 0.0, nx, ny, qM, qp);
+      if (code < 0) boundary_state<EQN>(*a.bc, -code - 1, 0.0, 0.0, 0.0, nx, ny, qM, qp);
       double lam;
       ef |= num_flux<EQN, FLUX>(a.ph, nx, ny, qM, qp, fs, &lam);
       lmax = lam > lmax ? lam : lmax;

@@ -16,6 +16,7 @@
 #include "../../include/apollo_dg.h"
 #include "apl_adjoint.h"
 #include "apl_device.h"
+#include "apl_eo.h"
 #include "apl_limiter.h"
 #include "apl_host.h"
 
@@ -37,7 +38,8 @@ struct apl_handle_s {
   apl_params params;
   int K = 0, M = 0, Nv = 0;
   bool linear = false;   // nodal linear-flux kernel (Maxwell, APL_ALGO_AUTO)
-  bool valu = false;     // cubature form on the VALU kernel (N <= 3)
+  bool valu = false;     // VALU kernel: cubature form (N <= 3, FP32) or nodal form
+  bool eo = false;       // cubature form on the even-odd kernel (FP64)
   Operators ops;
   Geometry geo;
   std::vector<int> etetf, fcode, vmapP;
@@ -49,6 +51,7 @@ struct apl_handle_s {
   // device buffers
   double *d_geom = nullptr, *d_vert = nullptr, *d_I1D = nullptr;
   int *d_fcode = nullptr, *d_fmask = nullptr;
+  BCTable *d_bc = nullptr;
   void *d_A1 = nullptr, *d_A2 = nullptr, *d_A3 = nullptr;
   unsigned *d_err = nullptr;
   double *d_speed = nullptr, *d_t = nullptr;
@@ -151,11 +154,13 @@ static int dev_alloc(apl_handle *h, void **dst, size_t bytes) {
   return APL_OK;
 }
 
-// The cubature form at N <= 3 (FP64 and FP32) runs on the VALU kernel
-// unless APL_ALGO_CUBATURE_MFMA asks for the MFMA kernel: measured faster
-// on the 2D Euler vortex at N = 3 (us per fused stage, VALU vs MFMA):
-// K = 8192 FP64 18.4 vs 20.4, FP32 15.4 vs 16.8; K = 131072 FP64 96.2 vs
-// 106.4, FP32 67.7 vs 75.2.
+// The cubature form in FP32 at N <= 3 runs on the VALU kernel unless
+// APL_ALGO_CUBATURE_MFMA asks for the MFMA kernel: measured faster on the 2D
+// Euler vortex at N = 3 (us per fused stage, VALU vs MFMA): K = 8192 15.4 vs
+// 16.8; K = 131072 67.7 vs 75.2.  In FP64 it runs on the even-odd kernel up
+// to this order: N = 3, K = 131072 68 us against 92 on the VALU kernel's FP64
+// form that it replaced, N = 4, K = 524288 404 against 585 on MFMA.
+constexpr int EO_MAX_ORDER = 4;
 constexpr bool VALU_BY_DEFAULT = true;
 // The nodal form of MAXWELL_TM3 runs on the VALU kernel under
 // APL_ALGO_AUTO (FP64 and FP32).
@@ -175,8 +180,8 @@ static int dispatch_rhs(apl_handle *h, const RhsArgs &a) {
   const int nb = (h->K + 15) / 16;
   const apl_params &p = h->params;
   // kernel: 0 cubature form on MFMA, 1 nodal form on MFMA, 2 cubature form
-  // on VALU, 3 nodal form on VALU
-  const int lin = h->linear ? (h->valu ? 3 : 1) : (h->valu ? 2 : 0);
+  // on VALU (FP32), 3 nodal form on VALU, 4 cubature form, even-odd (FP64)
+  const int lin = h->linear ? (h->valu ? 3 : 1) : h->eo ? 4 : (h->valu ? 2 : 0);
   int rc;
   switch (p.order) {
     case 1: rc = launch_rhs<1>(p.eqn, p.flux, p.precision, lin, h->stream, a, nb); break;
@@ -191,6 +196,53 @@ static int dispatch_rhs(apl_handle *h, const RhsArgs &a) {
   }
   if (rc) return fail(h, rc, "RHS kernel launch failed");
   return APL_OK;
+}
+
+// The boundary list as the kernels read it: inflow (wxeulerinflowbc.cc:21-36)
+// and Dirichlet (wxeulerdirichletbc.cc:22-30) states formed here.
+static BCTable bc_table(const apl_params &p) {
+  BCTable t;
+  t.n = p.n_bc;
+  for (int i = 0; i < APL_MAX_BC; ++i) {
+    t.kind[i] = p.bc[i].kind;
+    const double *s = p.bc[i].p;
+    double *d = t.p[i];
+    for (int j = 0; j < 8; ++j) d[j] = s[j];
+    double rho, u, v, w = 0.0, pres, g1;
+    if (p.bc[i].kind == APL_BC_EULER_INFLOW) {
+      const double pi = 3.141592653589793;
+      pres = s[3];
+      rho = s[4];
+      g1 = s[2] - 1;
+      const double sound = std::sqrt(s[2] * pres / rho);
+      u = s[0] * sound * std::cos(s[1] * pi / 180.);
+      v = s[0] * sound * std::sin(s[1] * pi / 180.);
+    } else if (p.bc[i].kind == APL_BC_EULER_DIRICHLET) {
+      rho = s[0];
+      u = s[1];
+      v = s[2];
+      w = s[3];
+      g1 = s[4] - 1;
+      pres = s[5];
+    } else {
+      continue;
+    }
+    t.kind[i] = BC_FIXED;
+    d[0] = rho;
+    d[1] = rho * u;
+    d[2] = rho * v;
+    d[3] = rho * w;
+    d[4] = pres / g1 + 0.5 * rho * (u * u + v * v + w * w);
+  }
+  return t;
+}
+
+// Whether a kernel reads the time: only the isentropic-vortex boundary
+// state depends on it.  Otherwise the captured step skips the clock kernel.
+static bool time_dependent(const apl_handle *h) {
+  for (int i = 0; i < h->params.n_bc; ++i)
+    if (h->params.bc[i].kind == APL_BC_ISENTROPIC_VORTEX) return true;
+  return false;
 }
 
 static RhsArgs base_args(apl_handle *h) {
@@ -213,11 +265,8 @@ static RhsArgs base_args(apl_handle *h) {
   a.ph.c0 = p.c0;
   a.ph.chi = p.chi;
   a.ph.gph = p.gamma_ph;
-  a.bc.n = p.n_bc;
-  for (int i = 0; i < APL_MAX_BC; ++i) {
-    a.bc.kind[i] = p.bc[i].kind;
-    for (int j = 0; j < 8; ++j) a.bc.p[i][j] = p.bc[i].p[j];
-  }
+  a.bc = h->d_bc;
+  a.vortex = time_dependent(h) ? 1 : 0;
   return a;
 }
 
@@ -301,7 +350,7 @@ static void make_fragments(const Operators &o, std::vector<T> &A1, std::vector<T
       }
 }
 
-// Point tables of the VALU cubature kernel (apl_valu.h): row c of A1 holds
+// Point tables of the VALU cubature kernel (apl_valu.h, FP32): row c of A1 holds
 // V_c[c, 0..Np), A_r[0..Np, c), A_s[0..Np, c); row k of A3 holds -L[0..Np, k).
 template <typename T>
 static void make_valu_tables(const Operators &o, std::vector<T> &A1, std::vector<T> &A3) {
@@ -318,6 +367,89 @@ static void make_valu_tables(const Operators &o, std::vector<T> &A1, std::vector
   A3.assign((size_t)3 * Ng * Np, T(0));
   for (int k = 0; k < 3 * Ng; ++k)
     for (int n = 0; n < Np; ++n) A3[(size_t)k * Np + n] = T(-L[(size_t)n * 3 * Ng + k]);
+}
+
+// Operator tables of the even-odd kernel (apl_eo.h).  False if the order's
+// nodes, faces or cubature rule do not have the mirror symmetry the kernel
+// is built on.
+static bool make_eo_tables(const Operators &o, std::vector<double> &A1, std::vector<double> &A2,
+                           std::vector<double> &A3) {
+  const int N = o.N, Np = o.Np, Nc = o.Nc, Ng = o.Ng, Nfp = o.Nfp;
+  const double tol = 1e-11;
+  for (int f = 0; f < 3; ++f)
+    for (int i = 0; i < Nfp; ++i)
+      if (o.fmask[f * Nfp + i] != eo_fmask(N, f, i)) return false;
+  std::vector<int> na, nb;   // node pairs, then the axis (EoNodes)
+  for (int j = 0; j <= N; ++j)
+    for (int i = j + 1; i + j <= N; ++i) {
+      na.push_back(eo_node(N, i, j));
+      nb.push_back(eo_node(N, j, i));
+    }
+  const int NO = (int)na.size();
+  for (int i = 0; 2 * i <= N; ++i) {
+    na.push_back(eo_node(N, i, i));
+    nb.push_back(eo_node(N, i, i));
+  }
+  const int NE = (int)na.size();
+  for (int i = 0; i < NE; ++i)
+    if (std::fabs(o.r[na[i]] - o.s[nb[i]]) + std::fabs(o.s[na[i]] - o.r[nb[i]]) > tol) return false;
+  std::vector<int> pc, pm, ax;   // point pairs and axis points
+  for (int c = 0; c < Nc; ++c) {
+    int m = -1;
+    for (int k = 0; k < Nc; ++k)
+      if (std::fabs(o.cr[c] - o.cs[k]) + std::fabs(o.cs[c] - o.cr[k]) < tol) m = k;
+    if (m < 0 || std::fabs(o.cw[c] - o.cw[m]) > tol) return false;
+    if (m == c) ax.push_back(c);
+    if (m > c) {
+      pc.push_back(c);
+      pm.push_back(m);
+    }
+  }
+  if ((int)ax.size() != eo_axis_points(N) || (int)(2 * pc.size() + ax.size()) != Nc) return false;
+  std::vector<double> Ar, As, L;
+  fold_operators(o, Ar, As, L);
+  // even and odd parts over the node list of a point's row (V) or column (A, L)
+  auto halves = [&](std::vector<double> &t, const double *x, int stride, double scale, bool even, bool odd) {
+    if (even)
+      for (int i = 0; i < NE; ++i)
+        t.push_back(scale * (i < NO ? 0.5 * (x[(size_t)na[i] * stride] + x[(size_t)nb[i] * stride])
+                                    : x[(size_t)na[i] * stride]));
+    if (odd)
+      for (int i = 0; i < NO; ++i)
+        t.push_back(scale * 0.5 * (x[(size_t)na[i] * stride] - x[(size_t)nb[i] * stride]));
+  };
+  A1.clear();
+  for (size_t p = 0; p < pc.size(); ++p) {
+    halves(A1, &o.Vc[(size_t)pc[p] * Np], 1, 1.0, true, true);
+    halves(A1, &Ar[pc[p]], Nc, 1.0, true, true);
+    halves(A1, &Ar[pm[p]], Nc, 1.0, true, true);
+  }
+  for (size_t p = 0; p < ax.size(); p += 2) {
+    const bool two = p + 1 < ax.size();   // a point left over goes with itself, weight zero
+    const int c1 = ax[p], c2 = two ? ax[p + 1] : c1;
+    halves(A1, &o.Vc[(size_t)c1 * Np], 1, 1.0, true, false);
+    halves(A1, &o.Vc[(size_t)c2 * Np], 1, 1.0, true, false);
+    halves(A1, &Ar[c1], Nc, 1.0, true, true);
+    halves(A1, &Ar[c2], Nc, two ? 1.0 : 0.0, true, true);
+  }
+  A3.clear();
+  for (int f = 0; f < 3; ++f)
+    for (int g = 0; g < Ng / 2; ++g) {
+      halves(A3, &L[f * Ng + g], 3 * Ng, -1.0, true, true);
+      halves(A3, &L[f * Ng + Ng - 1 - g], 3 * Ng, -1.0, true, true);
+    }
+  // the face interpolation is the same on the three faces; its even and odd
+  // parts per Gauss pair, then the abscissae
+  A2.clear();
+  for (int g = 0; g < Ng / 2; ++g) {
+    const double *x = &o.If[(size_t)g * Np];
+    auto at = [&](int i) { return x[o.fmask[i]]; };
+    for (int i = 0; i < (Nfp + 1) / 2; ++i)
+      A2.push_back(2 * i + 1 == Nfp ? at(i) : 0.5 * (at(i) + at(Nfp - 1 - i)));
+    for (int i = 0; i < Nfp / 2; ++i) A2.push_back(0.5 * (at(i) - at(Nfp - 1 - i)));
+  }
+  for (int g = 0; g < Ng / 2; ++g) A2.push_back(o.gz[g]);
+  return true;
 }
 
 // The folded operators of the nodal linear-flux form: D0 = Dt_r = A_r V_c,
@@ -420,6 +552,10 @@ static int upload_fragments(apl_handle *h) {
   } else if (h->linear) {
     make_linear_fragments<T>(h->ops, A1, A3, std::is_same<T, double>::value);
     A2.assign(1, T(0));
+  } else if (h->eo) {
+    if constexpr (std::is_same<T, double>::value)
+      if (!make_eo_tables(h->ops, A1, A2, A3))
+        return fail(h, APL_ERR_ORDER, "the order's tables lack the mirror symmetry");
   } else if (h->valu) {
     make_valu_tables<T>(h->ops, A1, A3);
     A2.assign(1, T(0));
@@ -521,7 +657,7 @@ static void free_graphs(apl_handle *h) {
 static void free_handle(apl_handle *h) {
   if (!h) return;
   free_graphs(h);
-  void *bufs[] = {h->d_geom, h->d_vert, h->d_I1D, h->d_fcode, h->d_fmask, h->d_A1, h->d_A2,
+  void *bufs[] = {h->d_bc, h->d_geom, h->d_vert, h->d_I1D, h->d_fcode, h->d_fmask, h->d_A1, h->d_A2,
                   h->d_A3, h->d_speed, h->d_t, h->d_qa, h->d_qb, h->d_res, h->d_out,
                   h->d_ckpt, h->d_Vc, h->d_cub, h->d_sbar, h->d_sbar2, h->d_qbar, h->d_rbar, h->d_stg,
                   h->d_seg, h->d_opart, h->d_lavg, h->d_lgrad, h->d_ltab, h->d_ltrc};
@@ -670,9 +806,11 @@ int apl_create(const apl_mesh *mesh, const apl_params *params, apl_handle **out)
               (params->algorithm == APL_ALGO_AUTO && NODAL_VALU_BY_DEFAULT &&
                params->eqn == APL_EQN_MAXWELL_TM3 && params->precision != APL_PREC_BF16X3);
   else
-    h->valu = params->order <= 3 && params->precision != APL_PREC_BF16X3 &&
+    h->valu = params->order <= 3 && params->precision == APL_PREC_FP32_MFMA &&
               (params->algorithm == APL_ALGO_CUBATURE_VALU ||
                (params->algorithm != APL_ALGO_CUBATURE_MFMA && VALU_BY_DEFAULT));
+  h->eo = !h->linear && params->precision == APL_PREC_FP64 && params->order <= EO_MAX_ORDER &&
+          params->algorithm != APL_ALGO_CUBATURE_MFMA;
   h->K = mesh->K;
   h->M = M;
   h->Nv = mesh->Nv;
@@ -764,6 +902,8 @@ int apl_create(const apl_mesh *mesh, const apl_params *params, apl_handle **out)
         I1D[((size_t)f * Ng + gq) * Nfp + i] = o.If[((size_t)f * Ng + gq) * Np + o.fmask[f * Nfp + i]];
   for (int gq = 0; gq < Ng; ++gq) I1D[(size_t)3 * Ng * Nfp + gq] = o.gz[gq];
 
+  const BCTable bct = bc_table(*params);
+  if ((rc = dev_upload<BCTable>(h, &h->d_bc, &bct, 1))) return bail(rc);
   if ((rc = dev_upload<double>(h, &h->d_geom, g.data(), g.size()))) return bail(rc);
   if ((rc = dev_upload<double>(h, &h->d_vert, h->geo.vert.data(), h->geo.vert.size()))) return bail(rc);
   if ((rc = dev_upload<int>(h, &h->d_fcode, h->fcode.data(), h->fcode.size()))) return bail(rc);
@@ -882,7 +1022,7 @@ static int enqueue_limit(apl_handle *h, const double *qin, double *qout, bool cl
   a.min_dens = h->params.lim_min_density;
   a.min_pres = h->params.lim_min_pressure;
   a.err = h->d_err;
-  a.bc = base_args(h).bc;
+  a.bc = h->d_bc;
   int rc;
   switch (h->params.order) {
     case 1: rc = launch_limiter<1>(h->params.eqn, h->stream, a); break;
@@ -1155,14 +1295,6 @@ static int enqueue_step(apl_handle *h, double *src, double *dst, double dt, bool
     if (launch_advance_time(h->stream, h->d_t, dt)) return fail(h, APL_ERR_HIP, "time kernel");
   }
   return APL_OK;
-}
-
-// Whether a kernel reads the time: only the isentropic-vortex boundary
-// state depends on it.  Otherwise the captured step skips the clock kernel.
-static bool time_dependent(const apl_handle *h) {
-  for (int i = 0; i < h->params.n_bc; ++i)
-    if (h->params.bc[i].kind == APL_BC_ISENTROPIC_VORTEX) return true;
-  return false;
 }
 
 static int build_graphs(apl_handle *h, double *qa, double *qb, double dt) {

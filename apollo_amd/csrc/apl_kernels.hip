@@ -3,6 +3,7 @@
 // orders build in parallel.
 #include "apl_adjoint.h"
 #include "apl_device.h"
+#include "apl_eo.h"
 #include "apl_limiter.h"
 #include "apl_valu.h"
 
@@ -29,9 +30,20 @@ static int launch_batches(K kern, hipStream_t s, const A &a, int nbatches) {
   return hipGetLastError() == hipSuccess ? APL_OK : APL_ERR_HIP;
 }
 
+// The even-odd kernel: groups of 32 elements, W waves each.
+template <int N, int EQN, int FLUX, int W, bool VTX = false>
+static int launch_eo(hipStream_t s, const RhsArgs &a) {
+  auto kern = rhs_eo_kernel<N, EQN, FLUX, W, VTX>;
+  const size_t lds = sizeof(double) * (size_t)EoCfg<N, EQN, W>::LDS;
+  if (!allow_lds(kern, lds)) return APL_ERR_UNSUPPORTED;
+  hipLaunchKernelGGL(kern, dim3((a.K + 31) / 32), dim3(64 * W), lds, s, a);
+  return hipGetLastError() == hipSuccess ? APL_OK : APL_ERR_HIP;
+}
+
 // kind: 0 the cubature form on MFMA, 1 the nodal form (linear fluxes) on
-// MFMA, 2 the cubature form on the VALU kernel (N <= 3, FP64 and FP32),
-// 3 the nodal form on the VALU kernel (TM, FP64 and FP32)
+// MFMA, 2 the cubature form on the VALU kernel (N <= 3, FP32), 3 the nodal
+// form on the VALU kernel (TM, FP64 and FP32), 4 the cubature form on the
+// even-odd kernel (N <= 4, FP64)
 template <int N, int EQN, int FLUX, typename T>
 static int launch_typed(int kind, hipStream_t s, const RhsArgs &a, int nblocks) {
   if constexpr (EQN == APL_EQN_PHMAXWELL8 || EQN == APL_EQN_MAXWELL_TM3) {
@@ -50,8 +62,28 @@ static int launch_typed(int kind, hipStream_t s, const RhsArgs &a, int nblocks) 
     }
   }
   if (kind == 1 || kind == 3) return APL_ERR_ARG;
+  if (kind == 4) {
+    if constexpr (N <= 4 && sizeof(T) == 8) {
+      if constexpr (EQN == APL_EQN_EULER5 || EQN == APL_EQN_EULER4)
+        if (a.vortex) return launch_eo<N, EQN, FLUX, 4, true>(s, a);
+      // One wave per group once the waves fill the card's 1024 SIMDs twice
+      // over (no reduction; us per stage, 1 against 4 waves: Euler N = 4,
+      // 16384 groups 404 / 494; 5-variable N = 4, 4096 groups 162 / 240);
+      // below that the last round of long waves costs more than the split
+      // (N = 3, 4096 groups 74 / 67; N = 4, 2500 groups 96 / 78).  Eight
+      // while a CU gets at most one group (256 groups, N = 4: 15.4 / 16.4
+      // with four).
+      const int groups = (a.K + 31) / 32;
+      if (groups >= 2 * 1024 * EoWaves<N, EQN, 1>::value) return launch_eo<N, EQN, FLUX, 1>(s, a);
+      if constexpr (EoCfg<N, EQN, 8>::LDS * 8 <= 163840)
+        if (groups <= 256) return launch_eo<N, EQN, FLUX, 8>(s, a);
+      return launch_eo<N, EQN, FLUX, 4>(s, a);
+    } else {
+      return APL_ERR_UNSUPPORTED;
+    }
+  }
   if (kind == 2) {
-    if constexpr (N <= 3 && sizeof(T) != 1) {
+    if constexpr (N <= 3 && sizeof(T) == 4) {
       // 64 elements per workgroup of four waves, or of eight on small meshes
       const int groups = (a.K + 63) / 64;
       if (groups < VALU_SMALL_GROUPS && ValuLds<N, EQN, T, 8>::doubles * 8 <= 163840) {

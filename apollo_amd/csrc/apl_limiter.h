@@ -84,7 +84,7 @@ struct LimArgs {
                            //          their ave-weighted means
   double gamma, min_dens, min_pres;
   unsigned *err;
-  BCTable bc;
+  const BCTable *bc;
 };
 
 // Limiter primitives (wxhesthavenwarburtoneulerlimiter.cc:535-543): no floors.
@@ -184,8 +184,11 @@ __global__ void __launch_bounds__(64) lim_average_kernel(LimArgs a) {
   }
 }
 
+// Two waves per SIMD: at three, which the registers (162) allow, more rows are
+// in flight than the L2 holds (K = 524288, N = 4: 263 -> 266 us per call).
 template <int N, int EQN>
-__global__ void __launch_bounds__(256) lim_gradient_kernel(LimArgs a) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+    lim_gradient_kernel(LimArgs a) {
   static_assert(N <= 4, "the reference's face-end reads leave its face array for N > 4");
   // at N = 1 each XCD takes one contiguous range of elements, so that most
   // neighbour rows are in its own L2 (K = 524288: 55.8 -> 50.3 us); at N = 4
@@ -262,9 +265,9 @@ __global__ void __launch_bounds__(256) lim_gradient_kernel(LimArgs a) {
       yc[f + 1] = yc[0] + 2.0 * gk[G_NY + f] * H1;
       A0[f + 1] = 0.0;
       const int bi = -code[f] - 1;
-      const int kind = (bi >= 0 && bi < a.bc.n) ? a.bc.kind[bi] : APL_BC_COPY;
-      const double *bp = a.bc.p[(bi >= 0 && bi < a.bc.n) ? bi : 0];
-      euler_bc5(kind, bp, 0.0, xc[f + 1], yc[f + 1], gk[G_NX + f], gk[G_NY + f], own, cf);
+      const int kind = (bi >= 0 && bi < a.bc->n) ? a.bc->kind[bi] : APL_BC_COPY;
+      const double *bp = a.bc->p[(bi >= 0 && bi < a.bc->n) ? bi : 0];
+      euler_bc5<false>(kind, bp, 0.0, xc[f + 1], yc[f + 1], gk[G_NX + f], gk[G_NY + f], own, cf);
     } else {
 #pragma unroll
       for (int c = 0; c < 5; ++c) cf[c] = av[f + 1][c];
@@ -288,9 +291,9 @@ __global__ void __launch_bounds__(256) lim_gradient_kernel(LimArgs a) {
       for (int c = 0; c < 5; ++c) qp[c] = qo[i][c];
     } else {
       const int bi = -cf - 1;
-      const int kind = (bi >= 0 && bi < a.bc.n) ? a.bc.kind[bi] : APL_BC_COPY;
-      const double *bp = a.bc.p[(bi >= 0 && bi < a.bc.n) ? bi : 0];
-      euler_bc5(kind, bp, 0.0, 0.0, 0.0, gk[G_NX + f], gk[G_NY + f], qo[i], qp);
+      const int kind = (bi >= 0 && bi < a.bc->n) ? a.bc->kind[bi] : APL_BC_COPY;
+      const double *bp = a.bc->p[(bi >= 0 && bi < a.bc->n) ? bi : 0];
+      euler_bc5<false>(kind, bp, 0.0, 0.0, 0.0, gk[G_NX + f], gk[G_NY + f], qo[i], qp);
     }
     double fc[5];
 #pragma unroll

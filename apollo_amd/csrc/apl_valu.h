@@ -1,4 +1,5 @@
-// apl_valu.h -- the cubature-form RHS on the vector ALU for N <= 3 (gfx950).
+// apl_valu.h -- the cubature-form RHS in FP32 on the vector ALU for N <= 3
+// (gfx950); FP64 runs on the even-odd kernel (apl_eo.h).
 //
 // The same RHS as rhs_kernel (apl_device.h), Apollo's over-integrated
 // cubature form (src/subsolvers/wxnodaldg2dmethod.cc:320-510,
@@ -83,16 +84,14 @@ struct ValuLds {
 // where their LDS fits a CU.
 constexpr int VALU_SMALL_GROUPS = 512;
 
-template <int N, int EQN, typename S>
-struct ValuWaves {
-  static constexpr int value = sizeof(S) == 8 ? 2 : 3;
-};
+// waves per SIMD asked of the register allocator
+constexpr int VALU_WAVES = 3;
 
 template <typename S>
 using cptr_t = const __attribute__((address_space(4))) S *;
 
 template <int N, int EQN, int FLUX, typename S, int W>
-__global__ void __launch_bounds__(64 * W, (ValuWaves<N, EQN, S>::value))
+__global__ void __launch_bounds__(64 * W, VALU_WAVES)
     rhs_valu_kernel(RhsArgs a) {
   using C = ValuCfg<N, EQN, W>;
   using L = ValuLds<N, EQN, S, W>;
@@ -100,7 +99,8 @@ __global__ void __launch_bounds__(64 * W, (ValuWaves<N, EQN, S>::value))
   constexpr int ES = C::ES, ESP = C::ESP, VW = C::VW, FW = C::FW, NFG = C::NFG;
   constexpr int NT = 64 * W;   // threads
   // FP32 face traces and flux where the FP32 MFMA kernel uses them
-  constexpr bool F32 = sizeof(S) == 4 && FLUX == APL_FLUX_LF && N <= 5 &&
+  static_assert(sizeof(S) == 4, "FP64 runs on the even-odd kernel");
+  constexpr bool F32 = FLUX == APL_FLUX_LF &&
                        (EQN == APL_EQN_EULER5 || EQN == APL_EQN_EULER4);
   typedef typename std::conditional<F32, float, double>::type TR;   // trace type
 
@@ -234,7 +234,7 @@ __global__ void __launch_bounds__(64 * W, (ValuWaves<N, EQN, S>::value))
           double dM[M], dP[M];
 #pragma unroll
           for (int v = 0; v < M; ++v) dM[v] = qM[v];
-          boundary_state<EQN>(a.bc, -code - 1, tnow, xg, yg, nx, ny, dM, dP);
+          boundary_state<EQN>(*a.bc, -code - 1, tnow, xg, yg, nx, ny, dM, dP);
 #pragma unroll
           for (int v = 0; v < M; ++v) qP[v] = float(dP[v]);
         }
@@ -259,7 +259,7 @@ __global__ void __launch_bounds__(64 * W, (ValuWaves<N, EQN, S>::value))
           const double sz = 0.5 * (1.0 + I1c[3 * Ng * Nfp + g]);
           const double xg = vk[2 * va] + sz * (vk[2 * vb] - vk[2 * va]);
           const double yg = vk[2 * va + 1] + sz * (vk[2 * vb + 1] - vk[2 * va + 1]);
-          boundary_state<EQN>(a.bc, -code - 1, tnow, xg, yg, nx, ny, qM, qP);
+          boundary_state<EQN>(*a.bc, -code - 1, tnow, xg, yg, nx, ny, qM, qP);
         }
         double fs[M], lam;
         ef |= num_flux<EQN, FLUX>(a.ph, nx, ny, qM, qP, fs, &lam);
@@ -299,18 +299,10 @@ __global__ void __launch_bounds__(64 * W, (ValuWaves<N, EQN, S>::value))
       }
       S F[M], G[M], phr[M], phs[M];
       ef |= phys_flux<EQN, S>(a.ph, qc, F, G);
-      if constexpr (sizeof(S) == 4) {
 #pragma unroll
-        for (int v = 0; v < M; ++v) {
-          phr[v] = jrx_s * F[v] + jry_s * G[v];
-          phs[v] = jsx_s * F[v] + jsy_s * G[v];
-        }
-      } else {
-#pragma unroll
-        for (int v = 0; v < M; ++v) {
-          phr[v] = S(jrx * double(F[v]) + jry * double(G[v]));
-          phs[v] = S(jsx * double(F[v]) + jsy * double(G[v]));
-        }
+      for (int v = 0; v < M; ++v) {
+        phr[v] = jrx_s * F[v] + jry_s * G[v];
+        phs[v] = jsx_s * F[v] + jsy_s * G[v];
       }
 #pragma unroll
       for (int n = 0; n < Np; ++n) {
@@ -519,7 +511,7 @@ __global__ void __launch_bounds__((64 * ValuLinCfg<N, EQN>::W), (ValuLinWaves<N,
 #pragma unroll
       for (int v = 0; v < M; ++v) qP[v] = src[v];
     } else {
-      boundary_state<EQN>(a.bc, -code - 1, 0.0, 0.0, 0.0, nx, ny, qM, qP);
+      boundary_state<EQN>(*a.bc, -code - 1, 0.0, 0.0, 0.0, nx, ny, qM, qP);
     }
     double lam;
     ef |= num_flux<EQN, FLUX>(a.ph, nx, ny, qM, qP, fs, &lam);

@@ -91,17 +91,16 @@ enum apl_algorithm {
                               identical nodal form V V^T Dr_c^T W V_c Q ... on
                               straight-sided elements (no reference
                               counterpart; same result to rounding).  The
-                              cubature form runs on the vector-ALU kernel at
-                              N <= 3 in FP64 and FP32, on MFMA otherwise     */
+                              cubature form runs on the vector ALU at N <= 4
+                              in FP64 and N <= 3 in FP32, on MFMA otherwise  */
   APL_ALGO_CUBATURE = 1,   /* always Apollo's over-integrated cubature form
                               (wxcubature2d.cc:288-382), on the kernels
                               APL_ALGO_AUTO picks for it                     */
   APL_ALGO_CUBATURE_MFMA = 2, /* the cubature form on the MFMA kernel at every
                               order (padded 16x16x4 tiles at N <= 3)         */
-  APL_ALGO_CUBATURE_VALU = 3, /* the cubature form on the vector-ALU kernel
-                              (one lane per element, operators as scalar
-                              operands); N <= 3, FP64 or FP32 only, else
-                              APL_ERR_UNSUPPORTED                            */
+  APL_ALGO_CUBATURE_VALU = 3, /* the cubature form on the vector-ALU kernels
+                              (operators as scalar operands); N <= 3, FP64
+                              or FP32 only, else APL_ERR_UNSUPPORTED         */
   APL_ALGO_NODAL_MFMA = 4, /* the nodal form of the linear fluxes on the MFMA
                               kernel (Maxwell only, else APL_ERR_ARG)        */
   APL_ALGO_NODAL_VALU = 5  /* the nodal form on the vector-ALU kernel (one
