@@ -1,4 +1,6 @@
-// apl_adjoint.h -- discrete adjoint of the cubature-form RHS (FP64, gfx950).
+// apl_adjoint.h -- discrete adjoint of the cubature-form RHS (FP64, gfx950):
+// its vector-Jacobian products, its MFMA kernels, and the objective.  The lower
+// orders run on the even-odd kernels (apl_adj_eo.h).
 //
 // No counterpart in the reference.  For rhs = (1/J)[A_r Phi_r + A_s Phi_s -
 // L S] (apl_device.h), the transpose applied to lam is, per element,
@@ -44,6 +46,7 @@ struct AdjArgs {
   const double *Avct;       // V_c^T fragments      [NRT][NCH][64][4] (acc_row permuted)
   const double *Alt;        // -L^T fragments       [NFT][NKS1][64]
   const double *Aift;       // I_f^T fragments      [NRT][NKF][64]
+  const double *TP, *TI, *TV;   // tables of the even-odd kernels (apl_adj_eo.h)
   double *sbar_out;         // mode 1: the next stage's Sb (kernel B), or null
   int face_pass;            // 1: kernel A computes Sb before kernel B runs
   double t;                 // time of the stage (boundary states)
@@ -52,6 +55,7 @@ struct AdjArgs {
   unsigned *err;
   PhysParams ph;
   const BCTable *bc;
+  int vortex;               // some boundary is the isentropic vortex
 };
 
 template <int N>

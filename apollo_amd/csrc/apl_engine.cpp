@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "../../include/apollo_dg.h"
+#include "apl_adj_eo.h"
 #include "apl_adjoint.h"
 #include "apl_device.h"
 #include "apl_eo.h"
@@ -64,6 +65,7 @@ struct apl_handle_s {
   // adjoint: FP64 operator fragments, work buffers, checkpoints
   double *d_adjops[6] = {nullptr};   // Avc, Aart, Aast, Avct, Alt, Aift
   double *d_Vc = nullptr, *d_cub = nullptr;
+  double *d_adjeo[3] = {nullptr};    // tables of the even-odd adjoint (TP, TI, TV)
   double *d_sbar = nullptr, *d_qbar = nullptr, *d_rbar = nullptr;
   double *d_sbar2 = nullptr;         // the reverse stepper's second face-weight buffer
   double *d_stg = nullptr;           // 2 stage buffers of forward_step
@@ -369,17 +371,8 @@ static void make_valu_tables(const Operators &o, std::vector<T> &A1, std::vector
     for (int n = 0; n < Np; ++n) A3[(size_t)k * Np + n] = T(-L[(size_t)n * 3 * Ng + k]);
 }
 
-// Operator tables of the even-odd kernel (apl_eo.h).  False if the order's
-// nodes, faces or cubature rule do not have the mirror symmetry the kernel
-// is built on.
-static bool make_eo_tables(const Operators &o, std::vector<double> &A1, std::vector<double> &A2,
-                           std::vector<double> &A3) {
-  const int N = o.N, Np = o.Np, Nc = o.Nc, Ng = o.Ng, Nfp = o.Nfp;
-  const double tol = 1e-11;
-  for (int f = 0; f < 3; ++f)
-    for (int i = 0; i < Nfp; ++i)
-      if (o.fmask[f * Nfp + i] != eo_fmask(N, f, i)) return false;
-  std::vector<int> na, nb;   // node pairs, then the axis (EoNodes)
+// The node pairs (na, nb), then the axis nodes (EoNodes); the number of pairs.
+static int eo_node_list(int N, std::vector<int> &na, std::vector<int> &nb) {
   for (int j = 0; j <= N; ++j)
     for (int i = j + 1; i + j <= N; ++i) {
       na.push_back(eo_node(N, i, j));
@@ -390,7 +383,21 @@ static bool make_eo_tables(const Operators &o, std::vector<double> &A1, std::vec
     na.push_back(eo_node(N, i, i));
     nb.push_back(eo_node(N, i, i));
   }
-  const int NE = (int)na.size();
+  return NO;
+}
+
+// Operator tables of the even-odd kernel (apl_eo.h).  False if the order's
+// nodes, faces or cubature rule do not have the mirror symmetry the kernel
+// is built on.
+static bool make_eo_tables(const Operators &o, std::vector<double> &A1, std::vector<double> &A2,
+                           std::vector<double> &A3) {
+  const int N = o.N, Np = o.Np, Nc = o.Nc, Ng = o.Ng, Nfp = o.Nfp;
+  const double tol = 1e-11;
+  for (int f = 0; f < 3; ++f)
+    for (int i = 0; i < Nfp; ++i)
+      if (o.fmask[f * Nfp + i] != eo_fmask(N, f, i)) return false;
+  std::vector<int> na, nb;
+  const int NO = eo_node_list(N, na, nb), NE = (int)na.size();
   for (int i = 0; i < NE; ++i)
     if (std::fabs(o.r[na[i]] - o.s[nb[i]]) + std::fabs(o.s[na[i]] - o.r[nb[i]]) > tol) return false;
   std::vector<int> pc, pm, ax;   // point pairs and axis points
@@ -665,6 +672,8 @@ static void free_handle(apl_handle *h) {
     if (b) (void)hipFree(b);
   if (h->h_pin) (void)hipHostFree(h->h_pin);
   for (double *b : h->d_adjops)
+    if (b) (void)hipFree(b);
+  for (double *b : h->d_adjeo)
     if (b) (void)hipFree(b);
   if (h->own_stream && h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
@@ -1446,8 +1455,7 @@ int apl_ssp_advance(apl_handle *h, double t0, double t_end, double dt0, double c
 // ---------------------------------------------------------------------------
 
 // FP64 fragments of the transposed operators (see apl_adjoint.h).
-static int ensure_adjoint_ops(apl_handle *h) {
-  if (h->d_adjops[0]) return APL_OK;
+static int upload_adjoint_fragments(apl_handle *h) {
   const Operators &o = h->ops;
   const int Np = o.Np, Nc = o.Nc, Ng = o.Ng;
   const int NKS1 = (Np + 3) / 4, NCH = (Nc + 15) / 16, NRT = (Np + 15) / 16, NKF = (3 * Ng + 3) / 4;
@@ -1507,6 +1515,40 @@ static int ensure_adjoint_ops(apl_handle *h) {
   int rc;
   for (int i = 0; i < 6; ++i)
     if ((rc = dev_upload<double>(h, &h->d_adjops[i], src[i]->data(), src[i]->size()))) return rc;
+  return APL_OK;
+}
+
+// Tables of the even-odd adjoint kernels (apl_adj_eo.h): the point rows of
+// apl_eo.h, its face interpolation with the Gauss weights, and V V^T on even
+// and odd parts.
+static int upload_adjoint_eo(apl_handle *h) {
+  const Operators &o = h->ops;
+  std::vector<double> A1, A2, A3, TV;
+  if (!make_eo_tables(o, A1, A2, A3)) return fail(h, APL_ERR_ORDER, "the order's tables lack the mirror symmetry");
+  for (int g = 0; g < o.Ng / 2; ++g) A2.push_back(o.gw[g]);
+  std::vector<int> na, nb;
+  const int NO = eo_node_list(o.N, na, nb), NE = (int)na.size();
+  const double *V = o.VVT.data();
+  for (int i = 0; i < NE; ++i)
+    for (int j = 0; j < NE; ++j)
+      TV.push_back(0.5 * (V[(size_t)na[i] * o.Np + na[j]] + V[(size_t)na[i] * o.Np + nb[j]]));
+  for (int i = 0; i < NO; ++i)
+    for (int j = 0; j < NO; ++j)
+      TV.push_back(0.5 * (V[(size_t)na[i] * o.Np + na[j]] - V[(size_t)na[i] * o.Np + nb[j]]));
+  const std::vector<double> *src[3] = {&A1, &A2, &TV};
+  int rc;
+  for (int i = 0; i < 3; ++i)
+    if ((rc = dev_upload<double>(h, &h->d_adjeo[i], src[i]->data(), src[i]->size()))) return rc;
+  return APL_OK;
+}
+
+static int ensure_adjoint_ops(apl_handle *h) {
+  if (h->d_Vc) return APL_OK;
+  const Operators &o = h->ops;
+  const int Np = o.Np, Nc = o.Nc, Ng = o.Ng;
+  const bool eo = adj_eo_order(o.N, h->M);
+  int rc;
+  if ((rc = eo ? upload_adjoint_eo(h) : upload_adjoint_fragments(h))) return rc;
   std::vector<double> cub((size_t)3 * Nc);
   for (int c = 0; c < Nc; ++c) {
     cub[3 * c] = o.cr[c];
@@ -1516,8 +1558,11 @@ static int ensure_adjoint_ops(apl_handle *h) {
   if ((rc = dev_upload<double>(h, &h->d_Vc, o.Vc.data(), o.Vc.size()))) return rc;
   if ((rc = dev_upload<double>(h, &h->d_cub, cub.data(), cub.size()))) return rc;
   const size_t n = state_len(h);
-  if ((rc = dev_alloc(h, (void **)&h->d_sbar, sizeof(double) * (size_t)h->K * 3 * Ng * h->M))) return rc;
-  if ((rc = dev_alloc(h, (void **)&h->d_sbar2, sizeof(double) * (size_t)h->K * 3 * Ng * h->M))) return rc;
+  // what the faces read: mu at the nodes (even-odd kernels) or Sb at the
+  // Gauss points
+  const size_t fw = sizeof(double) * (size_t)h->K * (eo ? Np : 3 * Ng) * h->M;
+  if ((rc = dev_alloc(h, (void **)&h->d_sbar, fw))) return rc;
+  if ((rc = dev_alloc(h, (void **)&h->d_sbar2, fw))) return rc;
   if ((rc = dev_alloc(h, (void **)&h->d_qbar, sizeof(double) * n))) return rc;
   if ((rc = dev_alloc(h, (void **)&h->d_rbar, sizeof(double) * n))) return rc;
   if ((rc = dev_alloc(h, (void **)&h->d_stg, sizeof(double) * n * 2))) return rc;
@@ -1541,7 +1586,11 @@ static AdjArgs adj_args(apl_handle *h) {
   a.Avct = h->d_adjops[3];
   a.Alt = h->d_adjops[4];
   a.Aift = h->d_adjops[5];
+  a.TP = h->d_adjeo[0];
+  a.TI = h->d_adjeo[1];
+  a.TV = h->d_adjeo[2];
   a.err = h->d_err;
+  a.vortex = r.vortex;
   a.ph = r.ph;
   a.bc = r.bc;
   return a;

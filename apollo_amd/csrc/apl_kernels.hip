@@ -1,6 +1,7 @@
 // apl_kernels.hip -- instantiates the RHS kernels of one polynomial order.
 // Compiled once per order with -DAPL_ORDER=<N> (see Makefile), so the eight
 // orders build in parallel.
+#include "apl_adj_eo.h"
 #include "apl_adjoint.h"
 #include "apl_device.h"
 #include "apl_eo.h"
@@ -70,11 +71,13 @@ static int launch_typed(int kind, hipStream_t s, const RhsArgs &a, int nblocks) 
       // over (no reduction; us per stage, 1 against 4 waves: Euler N = 4,
       // 16384 groups 404 / 494; 5-variable N = 4, 4096 groups 162 / 240);
       // below that the last round of long waves costs more than the split
-      // (N = 3, 4096 groups 74 / 67; N = 4, 2500 groups 96 / 78).  Eight
+      // (N = 3, 4096 groups 74 / 67; N = 4, 2500 groups 96 / 78), unless a
+      // CU's LDS holds only one four-wave group.  Eight
       // while a CU gets at most one group (256 groups, N = 4: 15.4 / 16.4
       // with four).
       const int groups = (a.K + 31) / 32;
-      if (groups >= 2 * 1024 * EoWaves<N, EQN, 1>::value) return launch_eo<N, EQN, FLUX, 1>(s, a);
+      constexpr bool PAIR = 2 * EoCfg<N, EQN, 4>::LDS * 8 <= 163840;
+      if (groups >= (PAIR ? 2 * EoWaves<N, EQN, 1>::value : 1) * 1024) return launch_eo<N, EQN, FLUX, 1>(s, a);
       if constexpr (EoCfg<N, EQN, 8>::LDS * 8 <= 163840)
         if (groups <= 256) return launch_eo<N, EQN, FLUX, 8>(s, a);
       return launch_eo<N, EQN, FLUX, 4>(s, a);
@@ -142,8 +145,36 @@ int launch_rhs(int eqn, int flux, int prec, int linear, hipStream_t s, const Rhs
 
 template int launch_rhs<APL_ORDER>(int, int, int, int, hipStream_t, const RhsArgs &, int);
 
+template <int N, int EQN, int FLUX, int W, bool VTX = false>
+static int launch_adj_eo(hipStream_t s, const AdjArgs &a) {
+  auto kern = a.mode == 1 ? adj_eo_kernel<N, EQN, FLUX, W, true, VTX> : adj_eo_kernel<N, EQN, FLUX, W, false, VTX>;
+  const size_t lds = sizeof(double) * (size_t)AdjEoCfg<N, EQN, W>::LDS;
+  if (!allow_lds(kern, lds)) return APL_ERR_UNSUPPORTED;
+  hipLaunchKernelGGL(kern, dim3((a.K + 31) / 32), dim3(64 * W), lds, s, a);
+  return hipGetLastError() == hipSuccess ? APL_OK : APL_ERR_HIP;
+}
+
 template <int N, int EQN, int FLUX>
 static int launch_adjoint_typed(hipStream_t s, const AdjArgs &a, int nblocks) {
+  if constexpr (adj_eo_order(N, Vars<EQN>::M)) {
+    const int groups = (a.K + 31) / 32;
+    if (a.face_pass) {
+      hipLaunchKernelGGL((adj_mu_kernel<N, EQN>), dim3(groups), dim3(64), 0, s, a);
+      if (hipGetLastError() != hipSuccess) return APL_ERR_HIP;
+    }
+    if constexpr (EQN == APL_EQN_EULER5 || EQN == APL_EQN_EULER4)
+      if (a.vortex) return launch_adj_eo<N, EQN, FLUX, 4, true>(s, a);
+    // as launch_eo, with a later change to one wave, since the larger units
+    // make its last round longer (us, 1 against 4 waves: adjoint RHS, Euler
+    // N = 3, 4096 groups 133 / 122; 5-variable N = 3, 2500 groups, where
+    // four-wave groups fill a CU's LDS one at a time, 137 / 164)
+    constexpr bool PAIR = 2 * AdjEoCfg<N, EQN, 4>::LDS * 8 <= 163840;
+    if (groups >= (PAIR ? 3 * AdjEoWaves<N, EQN, 1>::value : 1) * 1024)
+      return launch_adj_eo<N, EQN, FLUX, 1>(s, a);
+    if constexpr (AdjEoCfg<N, EQN, 8>::LDS * 8 <= 163840)
+      if (groups <= 256) return launch_adj_eo<N, EQN, FLUX, 8>(s, a);
+    return launch_adj_eo<N, EQN, FLUX, 4>(s, a);
+  } else {
   if (a.face_pass) {
     const int rc = launch_batches<AdjFaceLds<N, EQN>::doubles, AdjFaceGroup<N, EQN>::W>(
         adj_face_kernel<N, EQN>, s, a, nblocks);
@@ -154,6 +185,7 @@ static int launch_adjoint_typed(hipStream_t s, const AdjArgs &a, int nblocks) {
         adj_rhs_kernel<N, EQN, FLUX, true>, s, a, nblocks);
   return launch_batches<AdjLds<N, EQN>::doubles, AdjGroup<N, EQN>::W>(
       adj_rhs_kernel<N, EQN, FLUX, false>, s, a, nblocks);
+  }
 }
 
 template <int N>

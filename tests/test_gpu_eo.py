@@ -96,3 +96,51 @@ def test_eo_reports_bad_states(N):
             eng.rhs(0.0, q, np.zeros_like(q))
         eng.close()
         assert e.value.status == status
+
+
+@pytest.mark.parametrize("n", [3, 4, 5, 40])
+@pytest.mark.parametrize("N,m", [(1, 4), (2, 5), (3, 5), (4, 4), (4, 3), (2, 8)])
+def test_eo_adjoint_sizes(n, N, m):
+    """The transposed RHS on a partial, an exact and several groups (eight
+    waves each), periodic (Euler) or with reflecting walls (Maxwell)."""
+    case = euler_case(n=n, N=N, m=m) if m in (4, 5) else maxwell_case(n=n, N=N, m=m, bc=E.BC_PEC)
+    _check_adjoint(case)
+
+
+@pytest.mark.parametrize("N,m,n,periodic", [(3, 4, 65, True), (4, 4, 182, True), (2, 4, 20, False),
+                                            (2, 4, 257, True)])
+def test_eo_adjoint_groups(N, m, n, periodic):
+    """Four-wave groups (n = 65, and the vortex boundary's), one-wave groups
+    where four-wave ones fill a CU's LDS (n = 182, 2071 groups) and where
+    they do not (n = 257, 4129 groups of four waves)."""
+    _check_adjoint(euler_case(n=n, N=N, m=m, periodic=periodic))
+
+
+def _check_adjoint(case):
+    q = case.state(amp=1e-3)
+    lam = np.random.default_rng(5).standard_normal(q.shape)
+    eng = E.Engine(case.mesh, case.params)
+    out = np.zeros_like(q)
+    eng.adjoint_rhs(0.3, q, lam, out)
+    eng.close()
+    with O.exact_geometry():
+        ref = from_oracle(case.params.eqn, O.adjoint_rhs(case.omesh, case.ophys, 0.3,
+                                                         to_oracle(case.params.eqn, q),
+                                                         to_oracle(case.params.eqn, lam)))
+    assert rel_l2(out, ref) <= 1e-12
+
+
+def test_eo_reverse_lserk4_partial_groups():
+    """Reverse stages whose next-stage weights cross a partial last group."""
+    case = euler_case(n=9, N=2, m=5, periodic=False)
+    q0 = case.state(amp=1e-3)
+    gT = np.random.default_rng(2).standard_normal(q0.shape)
+    eng = E.Engine(case.mesh, case.params)
+    g0, qT = np.zeros_like(q0), np.zeros_like(q0)
+    eng.lserk4_adjoint(0.2, 0.01, 3, 2, q0, gT, g0, qT)
+    eng.close()
+    with O.exact_geometry():
+        ref = from_oracle(case.params.eqn, O.lserk4_adjoint(case.omesh, case.ophys, 0.2, 0.01, 3,
+                                                            to_oracle(case.params.eqn, q0),
+                                                            to_oracle(case.params.eqn, gT)))
+    assert rel_l2(g0, ref) <= 1e-11
