@@ -1712,8 +1712,17 @@ __global__ void __launch_bounds__((64 * LinGroup<N, EQN, T>::W), (LinWaves<N, EQ
 // Advance the device clock by dt at the end of a captured step.
 int launch_advance_time(hipStream_t s, double *t, double dt);
 
-// out[0] = max(in[0 .. n)), one workgroup.
-int launch_max_reduce(hipStream_t s, const double *in, int n, double *out);
+// What a call reports, in one small kernel that writes to pinned host memory:
+// pin[0] = max(in[0 .. n)) (0 if n == 0), pin[1] = the error flags (an
+// unsigned), which it clears for the next call.
+int launch_report(hipStream_t s, const double *in, int n, unsigned *err, double *pin);
+
+// part[b] = the largest squared Roe speed of the nodes of workgroup b
+// (SPEED_BLOCKS of them at most; returns how many in *nparts), Euler with m
+// = 4 or 5 variables.
+constexpr int SPEED_BLOCKS = 1024;
+int launch_roe_speed(hipStream_t s, const double *q, long nodes, int m, double gamma, double *part,
+                     int *nparts);
 
 // Launch entry of one order (defined in apl_kernels_N<N>.hip); `linear`
 // selects the nodal kernel (Maxwell only).

@@ -79,8 +79,10 @@ struct apl_handle_s {
   double *d_lavg = nullptr, *d_lgrad = nullptr, *d_ltab = nullptr, *d_ltrc = nullptr;
   LimTrace ltr{};
   bool ltr_is_state = false;   // trace slots = nodes 0..Np-1 of a 5-variable state
-  // pinned host words the flag and speed read-backs land in (two doubles)
+  // pinned host words the speed maximum and the flags are reported to (two
+  // doubles); flags_set: kernels ran since the flags were last cleared
   double *h_pin = nullptr;
+  bool flags_set = true;
   // this device's copy of apl_rhs_noalloc's scratch array (not owned)
   double *scratch = nullptr;
   std::string scratch_error;
@@ -90,8 +92,8 @@ struct apl_handle_s {
 // the device scratch of apl_rhs_noalloc
 // ---------------------------------------------------------------------------
 // apl_rhs_noalloc uses this file-scope array instead of the handle's
-// buffers, so that it allocates nothing.  Layout in doubles: [0] the reduced
-// speed maximum, [1] the error flags (its low 32 bits), [2, 32) unused,
+// buffers, so that it allocates nothing.  Layout in doubles: [1] the error
+// flags (its low 32 bits), the rest of [0, 32) unused,
 // [32, 32 + nb) the per-batch speed maxima of one RHS over nb = ceil(K/16)
 // batches.  Every GPU the library runs on holds its own copy (8 MB) until
 // the process ends; calls that overlap on one GPU share it and race.
@@ -280,13 +282,23 @@ static int flags_status(apl_handle *h, unsigned ef) {
   return APL_OK;
 }
 
-// Read the error flags after everything enqueued so far (one stream
-// synchronisation).
-static int check_flags(apl_handle *h) {
-  unsigned *pf = (unsigned *)h->h_pin;
-  HIPCHK(h, hipMemcpyAsync(pf, h->d_err, sizeof(unsigned), hipMemcpyDeviceToHost, h->stream));
+// Before the first kernel of a call: the flags are zero (each report clears
+// them; only a call that ended before its report leaves them set).
+static int begin_flags(apl_handle *h) {
+  if (h->flags_set) HIPCHK(h, hipMemsetAsync(h->d_err, 0, sizeof(unsigned), h->stream));
+  h->flags_set = true;
+  return APL_OK;
+}
+
+// Status of everything enqueued so far, after one stream synchronisation;
+// *speed (optional) receives the largest of the n partial speeds `part`.
+static int report(apl_handle *h, const double *part = nullptr, int n = 0, double *speed = nullptr) {
+  if (launch_report(h->stream, part, n, h->d_err, h->h_pin))
+    return fail(h, APL_ERR_HIP, "report kernel launch failed");
   HIPCHK(h, hipStreamSynchronize(h->stream));
-  return flags_status(h, *pf);
+  h->flags_set = false;
+  if (speed) *speed = h->h_pin[0];
+  return flags_status(h, *(const unsigned *)(h->h_pin + 1));
 }
 
 // The folded operators of the cubature form: A_r = V V^T Dr_c^T diag(w)
@@ -927,9 +939,10 @@ int apl_create(const apl_mesh *mesh, const apl_params *params, apl_handle **out)
     h->last_error = "pinned host allocation failed";
     return bail(APL_ERR_HIP);
   }
-  if ((rc = dev_alloc(h, (void **)&h->d_speed, sizeof(double) * ((h->K + 15) / 16)))) return bail(rc);
-  // d_t: [0] device clock, [1] a step's speed maximum, [2] the error flags
-  // (an unsigned), so that one copy reads back both of a step's results
+  if ((rc = dev_alloc(h, (void **)&h->d_speed,
+                      sizeof(double) * std::max((h->K + 15) / 16, SPEED_BLOCKS))))
+    return bail(rc);
+  // d_t: [0] device clock, [2] the error flags (an unsigned)
   if ((rc = dev_alloc(h, (void **)&h->d_t, sizeof(double) * 4))) return bail(rc);
   h->d_err = (unsigned *)(h->d_t + 2);
   if (params->limiter) {
@@ -1009,9 +1022,7 @@ int apl_create(const apl_mesh *mesh, const apl_params *params, apl_handle **out)
 }
 
 // The limiter's three passes on the handle's stream (qout may equal qin).
-// clear_err: the first pass zeroes the error flags (apl_limit's own call;
-// the steppers keep the flags of the step's earlier kernels).
-static int enqueue_limit(apl_handle *h, const double *qin, double *qout, bool clear_err = false) {
+static int enqueue_limit(apl_handle *h, const double *qin, double *qout) {
   LimArgs a;
   a.K = h->K;
   a.qin = qin;
@@ -1024,7 +1035,6 @@ static int enqueue_limit(apl_handle *h, const double *qin, double *qout, bool cl
   a.trc = h->d_ltrc;
   a.trc_rd = h->ltr_is_state ? qin : h->d_ltrc;
   a.trc_write = h->ltr_is_state ? 0 : 1;
-  a.clear_err = clear_err ? 1 : 0;
   a.tr = h->ltr;
   a.tab = h->d_ltab;
   a.gamma = h->params.lim_gas_gamma;
@@ -1048,16 +1058,16 @@ int apl_limit(apl_handle *h, const double *q_in, double *q_out, int where) {
   if (!h || !q_in || !q_out) return APL_ERR_ARG;
   if (!h->params.limiter) return fail(h, APL_ERR_ARG, "apl_limit: handle created without the limiter");
   int rc;
-  if ((rc = ensure_work(h))) return rc;
+  if ((rc = ensure_work(h)) || (rc = begin_flags(h))) return rc;
   if (where == APL_HOST) {
     const size_t bytes = sizeof(double) * state_len(h);
     HIPCHK(h, hipMemcpyAsync(h->d_qa, q_in, bytes, hipMemcpyHostToDevice, h->stream));
-    if ((rc = enqueue_limit(h, h->d_qa, h->d_qa, true))) return rc;
+    if ((rc = enqueue_limit(h, h->d_qa, h->d_qa))) return rc;
     HIPCHK(h, hipMemcpyAsync(q_out, h->d_qa, bytes, hipMemcpyDeviceToHost, h->stream));
   } else {
-    if ((rc = enqueue_limit(h, q_in, q_out, true))) return rc;
+    if ((rc = enqueue_limit(h, q_in, q_out))) return rc;
   }
-  return check_flags(h);
+  return report(h);
 }
 
 int apl_destroy(apl_handle *h) {
@@ -1165,26 +1175,20 @@ int apl_rhs(apl_handle *h, double t, const double *q, double *rhs, double cfl,
     dq = h->d_qa;
     drhs = h->d_out;
   }
-  HIPCHK(h, hipMemsetAsync(h->d_err, 0, sizeof(unsigned), h->stream));
+  if ((rc = begin_flags(h))) return rc;
   RhsArgs a = base_args(h);
   a.mode = 0;
   a.q = dq;
   a.out = drhs;
   a.t = t;
-  a.speed_part = h->d_speed;
+  a.speed_part = suggested_dt ? h->d_speed : nullptr;
   if ((rc = dispatch_rhs(h, a))) return rc;
   if (where == APL_HOST)
     HIPCHK(h, hipMemcpyAsync(rhs, drhs, bytes, hipMemcpyDeviceToHost, h->stream));
-  if ((rc = check_flags(h))) return rc;
-  if (suggested_dt) {
-    const int nb = (h->K + 15) / 16;
-    std::vector<double> sp(nb);
-    HIPCHK(h, hipMemcpy(sp.data(), h->d_speed, sizeof(double) * nb, hipMemcpyDeviceToHost));
-    double ms = 0.0;
-    for (double s : sp) ms = s > ms ? s : ms;
-    // wxnodaldg2dmethod.cc:523
-    *suggested_dt = 2. / 3. * cfl * h->geo.dtscale * (h->ops.rmin / ms);
-  }
+  double ms = 0.0;
+  if ((rc = report(h, h->d_speed, suggested_dt ? (h->K + 15) / 16 : 0, &ms))) return rc;
+  // wxnodaldg2dmethod.cc:523
+  if (suggested_dt) *suggested_dt = 2. / 3. * cfl * h->geo.dtscale * (h->ops.rmin / ms);
   return APL_OK;
 }
 
@@ -1200,8 +1204,7 @@ int apl_rhs_noalloc(apl_handle *h, double t, const double *q, double *rhs, doubl
                                     std::to_string(16 * NOALLOC_MAX_BATCHES) + " elements");
   if (states_overlap(h, q, rhs))
     return fail(h, APL_ERR_ARG, "rhs_noalloc: the output overlaps the input state");
-  // the flags and the reduced maximum start at zero (the array keeps the
-  // last call's contents)
+  // the flags start at zero (a call that failed to launch may have left them)
   HIPCHK(h, hipMemsetAsync(h->scratch, 0, sizeof(double) * NOALLOC_HEAD, h->stream));
   RhsArgs a = base_args(h);
   a.mode = 0;
@@ -1212,39 +1215,39 @@ int apl_rhs_noalloc(apl_handle *h, double t, const double *q, double *rhs, doubl
   a.speed_part = h->scratch + NOALLOC_HEAD;
   int rc;
   if ((rc = dispatch_rhs(h, a))) return rc;
-  if (suggested_dt && launch_max_reduce(h->stream, h->scratch + NOALLOC_HEAD, (int)nb, h->scratch))
-    return fail(h, APL_ERR_HIP, "rhs_noalloc: max kernel");
-  double back[2];
-  HIPCHK(h, hipMemcpyAsync(back, h->scratch, sizeof(back), hipMemcpyDeviceToHost, h->stream));
+  if (launch_report(h->stream, h->scratch + NOALLOC_HEAD, suggested_dt ? (int)nb : 0, a.err, h->h_pin))
+    return fail(h, APL_ERR_HIP, "rhs_noalloc: report kernel");
   HIPCHK(h, hipStreamSynchronize(h->stream));
-  unsigned ef;
-  std::memcpy(&ef, &back[1], sizeof(ef));
-  if ((rc = flags_status(h, ef))) return rc;
+  if ((rc = flags_status(h, *(const unsigned *)(h->h_pin + 1)))) return rc;
   // wxnodaldg2dmethod.cc:523
-  if (suggested_dt) *suggested_dt = 2. / 3. * cfl * h->geo.dtscale * (h->ops.rmin / back[0]);
+  if (suggested_dt) *suggested_dt = 2. / 3. * cfl * h->geo.dtscale * (h->ops.rmin / h->h_pin[0]);
   return APL_OK;
 }
 
 int apl_initial_dt(apl_handle *h, const double *q, double cfl, double *dt, int where) {
   if (!h || !q || !dt) return APL_ERR_ARG;
-  const size_t n = state_len(h);
-  std::vector<double> hq;
-  const double *qq = q;
-  if (where == APL_DEVICE) {
-    hq.resize(n);
-    HIPCHK(h, hipMemcpy(hq.data(), q, sizeof(double) * n, hipMemcpyDeviceToHost));
-    qq = hq.data();
-  }
   // Roe speeds of the node state against itself (wxnodaldg2dmethod.cc:201-213,
   // wxeulereqn.cc:95-234); phMaxwell's fastest wave is c0 max(chi, gamma, 1).
   const apl_params &p = h->params;
   const int M = h->M;
+  const size_t nodes = state_len(h) / M;
   double maxSpeed = 0.0;
-  const bool euler = (p.eqn == APL_EQN_EULER5 || p.eqn == APL_EQN_EULER4);
-  for (size_t i = 0; i < n / M; ++i) {
-    const double *d = qq + i * M;
-    double lam = 0.0;
-    if (euler) {
+  if (p.eqn != APL_EQN_EULER5 && p.eqn != APL_EQN_EULER4) {
+    maxSpeed = std::max(std::max(p.chi * p.c0, p.gamma_ph * p.c0), p.c0);
+  } else if (where == APL_DEVICE) {
+    // q may come from the null stream, which a caller's own stream does not
+    // wait for
+    if (!h->own_stream) HIPCHK(h, hipStreamSynchronize(nullptr));
+    int n = 0;
+    if (launch_roe_speed(h->stream, q, (long)nodes, M, p.gas_gamma, h->d_speed, &n))
+      return fail(h, APL_ERR_HIP, "wave speed kernel launch failed");
+    int rc;
+    double s2 = 0.0;
+    if ((rc = begin_flags(h)) || (rc = report(h, h->d_speed, n, &s2))) return rc;
+    maxSpeed = std::sqrt(s2);
+  } else {
+    for (size_t i = 0; i < nodes; ++i) {
+      const double *d = q + i * M;
       const double rho = d[0], mu = d[1], mv = d[2];
       const double mw = (p.eqn == APL_EQN_EULER5) ? d[3] : 0.0;
       const double E = (p.eqn == APL_EQN_EULER5) ? d[4] : d[3];
@@ -1253,12 +1256,10 @@ int apl_initial_dt(apl_handle *h, const double *q, double cfl, double *dt, int w
       const double u = mu / rho, v = mv / rho, w = mw / rho;
       const double enth = (E + pr) / rho;
       const double a = std::sqrt(g1 * (enth - 0.5 * (u * u + v * v + w * w)));
+      double lam = 0.0;
       for (double s : {u - a, u, u + a, v - a, v, v + a}) lam = std::max(lam, s * s);
-      lam = std::sqrt(lam);
-    } else {
-      lam = std::max(std::max(p.chi * p.c0, p.gamma_ph * p.c0), p.c0);
+      maxSpeed = std::max(maxSpeed, std::sqrt(lam));
     }
-    maxSpeed = std::max(maxSpeed, lam);
   }
   *dt = 2. / 3. * cfl * h->geo.dtscale * (h->ops.rmin / maxSpeed);
   return APL_OK;
@@ -1286,7 +1287,7 @@ static int enqueue_step(apl_handle *h, double *src, double *dst, double dt, bool
   a.mode = 1;
   a.res = h->d_res;
   a.dt = dt;
-  a.tptr = h->d_t;
+  a.tptr = advance ? h->d_t : nullptr;
   a.speed_part = nullptr;
   double *bufs[2] = {src, dst};
   for (int s = 0; s < 5; ++s) {
@@ -1332,12 +1333,13 @@ static int run_lserk4(apl_handle *h, double t0, double dt, int nsteps, double *q
   int rc;
   if (h->graph_qa != qa || h->graph_dt != dt || !h->step_exec[0])
     if ((rc = build_graphs(h, qa, qb, dt))) return rc;
-  HIPCHK(h, hipMemcpyAsync(h->d_t, &t0, sizeof(double), hipMemcpyHostToDevice, h->stream));
-  HIPCHK(h, hipMemsetAsync(h->d_err, 0, sizeof(unsigned), h->stream));
+  if (time_dependent(h))
+    HIPCHK(h, hipMemcpyAsync(h->d_t, &t0, sizeof(double), hipMemcpyHostToDevice, h->stream));
+  if ((rc = begin_flags(h))) return rc;
   for (int s = 0; s < nsteps; ++s) HIPCHK(h, hipGraphLaunch(h->step_exec[s & 1], h->stream));
   if (nsteps & 1)
     HIPCHK(h, hipMemcpyAsync(qa, qb, sizeof(double) * state_len(h), hipMemcpyDeviceToDevice, h->stream));
-  return check_flags(h);
+  return report(h);
 }
 
 int apl_lserk4(apl_handle *h, double t0, double dt, int nsteps, double *q, int where) {
@@ -1385,8 +1387,7 @@ int apl_ssp_advance(apl_handle *h, double t0, double t_end, double dt0, double c
   }
   double *bufs[2] = {h->d_qb, h->d_res};
   const int nb = (h->K + 15) / 16;
-  double *d_smax = h->d_t + 1;
-  HIPCHK(h, hipMemsetAsync(h->d_err, 0, sizeof(unsigned), h->stream));
+  if ((rc = begin_flags(h))) return rc;
   RhsArgs a = base_args(h);
   a.mode = 2;
   double t = t0, dt_temp = dt0;
@@ -1432,12 +1433,9 @@ int apl_ssp_advance(apl_handle *h, double t0, double t_end, double dt0, double c
     a.t = t + dt;
     a.speed_part = h->d_speed;
     if ((rc = dispatch_rhs(h, a))) return rc;
-    if (launch_max_reduce(h->stream, h->d_speed, nb, d_smax)) return fail(h, APL_ERR_HIP, "max kernel");
-    // the speed maximum and the flags word after it, in one copy
-    HIPCHK(h, hipMemcpyAsync(h->h_pin, d_smax, 2 * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
-    const double ms = h->h_pin[0];
-    if (*(const unsigned *)(h->h_pin + 1)) return check_flags(h);
+    double ms = 0.0;
+    if ((rc = report(h, h->d_speed, nb, &ms))) return rc;
+    h->flags_set = true;   // the next step's kernels
     // wxnodaldg2dmethod.cc:523, then apsolver.cc:474
     const double suggested = 2. / 3. * cfl * h->geo.dtscale * (h->ops.rmin / ms);
     dt_temp = std::fmin(suggested, dt);
@@ -1445,9 +1443,10 @@ int apl_ssp_advance(apl_handle *h, double t0, double t_end, double dt0, double c
     if (dts) dts[n] = dt;
     ++n;
   }
+  h->flags_set = false;   // the last step's report cleared them
   if (nsteps) *nsteps = n;
   if (where == APL_HOST) HIPCHK(h, hipMemcpy(q, sol, bytes, hipMemcpyDeviceToHost));
-  return check_flags(h);
+  return APL_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -1635,7 +1634,7 @@ int apl_adjoint_rhs(apl_handle *h, double t, const double *q, const double *lam,
     dl = h->d_qb;
     dout = h->d_out;
   }
-  HIPCHK(h, hipMemsetAsync(h->d_err, 0, sizeof(unsigned), h->stream));
+  if ((rc = begin_flags(h))) return rc;
   AdjArgs a = adj_args(h);
   a.mode = 0;
   a.face_pass = 1;
@@ -1645,7 +1644,7 @@ int apl_adjoint_rhs(apl_handle *h, double t, const double *q, const double *lam,
   a.t = t;
   if ((rc = dispatch_adjoint(h, a))) return rc;
   if (where == APL_HOST) HIPCHK(h, hipMemcpyAsync(out, dout, bytes, hipMemcpyDeviceToHost, h->stream));
-  return check_flags(h);
+  return report(h);
 }
 
 // One forward LSERK4 step from `in` to `result`, its stage inputs
@@ -1724,7 +1723,7 @@ int apl_lserk4_adjoint(apl_handle *h, double t0, double dt, int nsteps, int ckpt
     h->seg_slots = nseg;
   }
   const hipMemcpyKind in_kind = where == APL_HOST ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
-  HIPCHK(h, hipMemsetAsync(h->d_err, 0, sizeof(unsigned), h->stream));
+  if ((rc = begin_flags(h))) return rc;
   // forward sweep with checkpoints; the steps of the last segment keep their
   // stage inputs in d_seg at once, so that segment needs no recompute
   const long long last = nsteps > 0 ? (nsteps - 1) / C : -1;
@@ -1796,7 +1795,7 @@ int apl_lserk4_adjoint(apl_handle *h, double t0, double dt, int nsteps, int ckpt
   }
   const hipMemcpyKind out_kind = where == APL_HOST ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice;
   HIPCHK(h, hipMemcpyAsync(dJdq0, h->d_qbar, bytes, out_kind, h->stream));
-  return check_flags(h);
+  return report(h);
 }
 
 int apl_objective_disc_sq(apl_handle *h, const double *q, int var, double xc, double yc,

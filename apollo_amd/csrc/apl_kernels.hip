@@ -279,25 +279,79 @@ int launch_advance_time(hipStream_t s, double *t, double dt) {
   return hipGetLastError() == hipSuccess ? APL_OK : APL_ERR_HIP;
 }
 
-// One 256-lane workgroup: strided maxima, then a tree over LDS.
-__global__ void __launch_bounds__(256) max_reduce_kernel(const double *in, int n, double *out) {
-  __shared__ double part[256];
+// One workgroup of 1024 lanes: strided maxima, eight loads of a lane in
+// flight at once, then a tree over LDS.  A host copy of the per-batch maxima
+// and of the flags took two transfers and two synchronisations (RHS of the
+// 8-variable Maxwell system, N = 4, K = 45000: 73 us per call, of which 48
+// the RHS kernel).
+__global__ void __launch_bounds__(1024) report_kernel(const double *in, int n, unsigned *err, double *pin) {
+  __shared__ double part[16];
   double m = 0.0;
-  for (int i = threadIdx.x; i < n; i += 256) m = in[i] > m ? in[i] : m;
-  part[threadIdx.x] = m;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) {
-      const double o = part[threadIdx.x + w];
-      part[threadIdx.x] = o > part[threadIdx.x] ? o : part[threadIdx.x];
-    }
-    __syncthreads();
+  for (int i = threadIdx.x; i < n; i += 8 * 1024) {
+    double v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = i + k * 1024 < n ? in[i + k * 1024] : 0.0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) m = v[k] > m ? v[k] : m;
   }
-  if (threadIdx.x == 0) out[0] = part[0];
+  for (int off = 32; off > 0; off >>= 1) {
+    const double o = __shfl_xor(m, off);
+    m = o > m ? o : m;
+  }
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < (int)blockDim.x / 64; ++w) m = part[w] > m ? part[w] : m;
+    pin[0] = m;
+    *(unsigned *)(pin + 1) = *err;
+    *err = 0u;
+  }
 }
 
-int launch_max_reduce(hipStream_t s, const double *in, int n, double *out) {
-  hipLaunchKernelGGL(max_reduce_kernel, dim3(1), dim3(256), 0, s, in, n, out);
+int launch_report(hipStream_t s, const double *in, int n, unsigned *err, double *pin) {
+  hipLaunchKernelGGL(report_kernel, dim3(1), dim3(n > 64 ? 1024 : 64), 0, s, in, n, err, pin);
+  return hipGetLastError() == hipSuccess ? APL_OK : APL_ERR_HIP;
+}
+
+// Roe speeds of each node's state against itself (wxnodaldg2dmethod.cc:201-213,
+// wxeulereqn.cc:95-234), squared, with the operations and the order of the
+// host's loop; a NaN speed does not count, as there.  A pass over the state,
+// bound by memory; on the host it took a copy of the state and a serial loop
+// (N = 1, K = 15842: 300 us, here 12).
+template <int M>
+__global__ void __launch_bounds__(256) roe_speed_kernel(const double *q, long nodes, double gamma, double *part) {
+#pragma clang fp contract(off)
+  __shared__ double wm[4];
+  const double g1 = gamma - 1.0;
+  double m = 0.0;
+  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < nodes; i += (long)gridDim.x * 256) {
+    const double *d = q + i * M;
+    const double rho = d[0], mu = d[1], mv = d[2], mw = M == 5 ? d[3] : 0.0, E = d[M - 1];
+    const double pr = g1 * (E - 0.5 * (mu * mu + mv * mv + mw * mw) / rho);
+    const double u = mu / rho, v = mv / rho, w = mw / rho;
+    const double enth = (E + pr) / rho;
+    const double a = sqrt(g1 * (enth - 0.5 * (u * u + v * v + w * w)));
+    const double s[6] = {u - a, u, u + a, v - a, v, v + a};
+#pragma unroll
+    for (int k = 0; k < 6; ++k) m = m < s[k] * s[k] ? s[k] * s[k] : m;
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    const double o = __shfl_xor(m, off);
+    m = o > m ? o : m;
+  }
+  if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int k = 1; k < 4; ++k) m = wm[k] > m ? wm[k] : m;
+    part[blockIdx.x] = m;
+  }
+}
+
+int launch_roe_speed(hipStream_t s, const double *q, long nodes, int m, double gamma, double *part, int *nparts) {
+  const int nb = (int)((nodes + 255) / 256 < SPEED_BLOCKS ? (nodes + 255) / 256 : SPEED_BLOCKS);
+  if (m == 5) hipLaunchKernelGGL(roe_speed_kernel<5>, dim3(nb), dim3(256), 0, s, q, nodes, gamma, part);
+  else hipLaunchKernelGGL(roe_speed_kernel<4>, dim3(nb), dim3(256), 0, s, q, nodes, gamma, part);
+  *nparts = nb;
   return hipGetLastError() == hipSuccess ? APL_OK : APL_ERR_HIP;
 }
 #endif
