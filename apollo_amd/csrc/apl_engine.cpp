@@ -1836,14 +1836,12 @@ int apl_objective_disc_sq(apl_handle *h, const double *q, int var, double xc, do
     default: rc = APL_ERR_ORDER;
   }
   if (rc) return fail(h, rc, "objective kernel launch failed");
-  std::vector<double> part(nb);
-  HIPCHK(h, hipMemcpyAsync(part.data(), h->d_opart, sizeof(double) * nb, hipMemcpyDeviceToHost, h->stream));
+  if (launch_sum_report(h->stream, h->d_opart, nb, h->h_pin))
+    return fail(h, APL_ERR_HIP, "objective sum launch failed");
   if (dJdq && where == APL_HOST)
     HIPCHK(h, hipMemcpyAsync(dJdq, h->d_out, bytes, hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
-  double sum = 0.0;
-  for (double v : part) sum += v;     // fixed order: deterministic
-  *J = sum;
+  *J = h->h_pin[0];
   return APL_OK;
 }
 

@@ -313,6 +313,25 @@ int launch_report(hipStream_t s, const double *in, int n, unsigned *err, double 
   return hipGetLastError() == hipSuccess ? APL_OK : APL_ERR_HIP;
 }
 
+// One workgroup: strided sums, then a tree; the same order on every call.
+__global__ void __launch_bounds__(1024) sum_report_kernel(const double *in, int n, double *pin) {
+  __shared__ double part[16];
+  double m = 0.0;
+  for (int i = threadIdx.x; i < n; i += 1024) m += in[i];
+  for (int off = 32; off > 0; off >>= 1) m += __shfl_xor(m, off);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 16; ++w) m += part[w];
+    pin[0] = m;
+  }
+}
+
+int launch_sum_report(hipStream_t s, const double *in, int n, double *pin) {
+  hipLaunchKernelGGL(sum_report_kernel, dim3(1), dim3(1024), 0, s, in, n, pin);
+  return hipGetLastError() == hipSuccess ? APL_OK : APL_ERR_HIP;
+}
+
 // Roe speeds of each node's state against itself (wxnodaldg2dmethod.cc:201-213,
 // wxeulereqn.cc:95-234), squared, with the operations and the order of the
 // host's loop; a NaN speed does not count, as there.  A pass over the state,
