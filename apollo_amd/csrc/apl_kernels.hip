@@ -313,18 +313,50 @@ int launch_report(hipStream_t s, const double *in, int n, unsigned *err, double 
   return hipGetLastError() == hipSuccess ? APL_OK : APL_ERR_HIP;
 }
 
-// One workgroup: strided sums, then a tree; the same order on every call.
+// One workgroup: the sum in index order, as a loop over the array rounds it.
+// Most partials of a disc's objective are zero and change no sum, so each wave
+// packs the others of its 256 to the front of LDS in their order, and one
+// thread's chain of dependent additions runs over those alone.  (A strided
+// sum with a tree is no shorter for a disc of 100 partials among 2048.)
 __global__ void __launch_bounds__(1024) sum_report_kernel(const double *in, int n, double *pin) {
-  __shared__ double part[16];
-  double m = 0.0;
-  for (int i = threadIdx.x; i < n; i += 1024) m += in[i];
-  for (int off = 32; off > 0; off >>= 1) m += __shfl_xor(m, off);
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < 16; ++w) m += part[w];
-    pin[0] = m;
+  __shared__ double val[4096];
+  __shared__ int cnt[16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double sum = 0.0;
+  for (int b = 0; b < n; b += 4096) {
+    double v[4];
+    unsigned long long some[4];
+    int mine = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int i = b + wave * 256 + j * 64 + lane;
+      v[j] = i < n ? in[i] : 0.0;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      some[j] = __ballot(!(v[j] == 0.0));
+      mine += __popcll(some[j]);
+    }
+    if (lane == 0) cnt[wave] = mine;
+    __syncthreads();
+    int at = 0, all = 0;
+    for (int w = 0; w < 16; ++w) {
+      if (w < wave) at += cnt[w];
+      all += cnt[w];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (some[j] >> lane & 1) val[at + __popcll(some[j] & ((1ull << lane) - 1))] = v[j];
+      at += __popcll(some[j]);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll 8
+      for (int i = 0; i < all; ++i) sum += val[i];
+    }
+    __syncthreads();
   }
+  if (threadIdx.x == 0) pin[0] = sum;
 }
 
 int launch_sum_report(hipStream_t s, const double *in, int n, double *pin) {
