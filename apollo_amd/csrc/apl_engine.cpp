@@ -18,6 +18,7 @@
 #include "apl_adjoint.h"
 #include "apl_device.h"
 #include "apl_eo.h"
+#include "apl_eo_linear.h"
 #include "apl_limiter.h"
 #include "apl_host.h"
 
@@ -40,7 +41,7 @@ struct apl_handle_s {
   int K = 0, M = 0, Nv = 0;
   bool linear = false;   // nodal linear-flux kernel (Maxwell, APL_ALGO_AUTO)
   bool valu = false;     // VALU kernel: cubature form (N <= 3, FP32) or nodal form
-  bool eo = false;       // cubature form on the even-odd kernel (FP64)
+  bool eo = false;       // on an even-odd kernel (FP64): rhs_eo_kernel, or rhs_eo_linear_kernel if linear
   Operators ops;
   Geometry geo;
   std::vector<int> etetf, fcode, vmapP;
@@ -184,8 +185,9 @@ static int dispatch_rhs(apl_handle *h, const RhsArgs &a) {
   const int nb = (h->K + 15) / 16;
   const apl_params &p = h->params;
   // kernel: 0 cubature form on MFMA, 1 nodal form on MFMA, 2 cubature form
-  // on VALU (FP32), 3 nodal form on VALU, 4 cubature form, even-odd (FP64)
-  const int lin = h->linear ? (h->valu ? 3 : 1) : h->eo ? 4 : (h->valu ? 2 : 0);
+  // on VALU (FP32), 3 nodal form on VALU, 4 cubature form, even-odd (FP64),
+  // 5 nodal form, even-odd (FP64)
+  const int lin = h->linear ? (h->valu ? 3 : h->eo ? 5 : 1) : h->eo ? 4 : (h->valu ? 2 : 0);
   int rc;
   switch (p.order) {
     case 1: rc = launch_rhs<1>(p.eqn, p.flux, p.precision, lin, h->stream, a, nb); break;
@@ -562,6 +564,73 @@ static void make_linear_fragments(const Operators &o, std::vector<T> &A1, std::v
       }
 }
 
+// Operator tables of the even-odd nodal kernel (apl_eo_linear.h): A1 the volume
+// rows, A3 the lift rows, A2 the units' node lists (ints).  False as
+// make_eo_tables.
+static bool make_eo_linear_tables(const Operators &o, std::vector<double> &A1,
+                                  std::vector<int> &A2, std::vector<double> &A3) {
+  const int N = o.N, Np = o.Np, Nfp = o.Nfp;
+  {
+    std::vector<double> t1, t2, t3;
+    if (!make_eo_tables(o, t1, t2, t3)) return false;
+  }
+  std::vector<int> na, nb;
+  const int NO = eo_node_list(N, na, nb), NE = (int)na.size();
+  std::vector<double> D[2], Lt;
+  fold_linear_operators(o, D, Lt);
+  auto rows = [&](std::vector<double> &t, const double *x, int stride, double se, double so) {
+    for (int i = 0; i < NE; ++i)
+      t.push_back(se * 0.5 * (x[(size_t)na[i] * stride] + x[(size_t)nb[i] * stride]));
+    for (int i = 0; i < NO; ++i)
+      t.push_back(so * 0.5 * (x[(size_t)na[i] * stride] - x[(size_t)nb[i] * stride]));
+  };
+  const int ppu = EO_LPE / 2;
+  A1.clear();
+  A2.clear();
+  A3.clear();
+  // volume pairs: node a, its mirror b (an axis node goes with itself, the
+  // second time with weight zero), padded to whole units
+  for (int p = 0; p < (NE + ppu - 1) / ppu * ppu; ++p) {
+    const int a = p < NE ? na[p] : 0, b = p < NE ? nb[p] : 0;
+    const double s1 = p < NE ? 1.0 : 0.0, s2 = p < NO ? 1.0 : 0.0;
+    rows(A1, &D[0][a], Np, s1, s1);
+    rows(A1, &D[0][b], Np, s2, s2);
+    A2.push_back(a);
+    A2.push_back(b);
+  }
+  // face-node pairs: bottom node i with left-side node N - i; hypotenuse node
+  // i with N - i (the middle one with itself, at half weight)
+  const int NLP = Nfp + (Nfp + 1) / 2;
+  for (int p = 0; p < (NLP + ppu - 1) / ppu * ppu; ++p) {
+    int k = 0, m = 0;
+    double s = 0.0;
+    if (p < Nfp) {
+      k = p;
+      m = 2 * Nfp + N - p;
+      s = 1.0;
+    } else if (p < NLP) {
+      k = Nfp + (p - Nfp);
+      m = Nfp + N - (p - Nfp);
+      s = k == m ? 0.5 : 1.0;
+    }
+    rows(A3, &Lt[k], 3 * Nfp, -s, -s);
+    A2.push_back(k);
+    A2.push_back(m);
+  }
+  return true;
+}
+
+static int upload_eo_linear(apl_handle *h) {
+  std::vector<double> A1, A3;
+  std::vector<int> A2;
+  if (!make_eo_linear_tables(h->ops, A1, A2, A3))
+    return fail(h, APL_ERR_ORDER, "the order's tables lack the mirror symmetry");
+  int rc;
+  if ((rc = dev_upload<double>(h, (double **)&h->d_A1, A1.data(), A1.size()))) return rc;
+  if ((rc = dev_upload<int>(h, (int **)&h->d_A2, A2.data(), A2.size()))) return rc;
+  return dev_upload<double>(h, (double **)&h->d_A3, A3.data(), A3.size());
+}
+
 template <typename T>
 static int upload_fragments(apl_handle *h) {
   std::vector<T> A1, A2, A3;
@@ -830,8 +899,10 @@ int apl_create(const apl_mesh *mesh, const apl_params *params, apl_handle **out)
     h->valu = params->order <= 3 && params->precision == APL_PREC_FP32_MFMA &&
               (params->algorithm == APL_ALGO_CUBATURE_VALU ||
                (params->algorithm != APL_ALGO_CUBATURE_MFMA && VALU_BY_DEFAULT));
-  h->eo = !h->linear && params->precision == APL_PREC_FP64 && params->order <= EO_MAX_ORDER &&
-          params->algorithm != APL_ALGO_CUBATURE_MFMA;
+  h->eo = params->precision == APL_PREC_FP64 &&
+          (h->linear ? params->algorithm == APL_ALGO_AUTO && !h->valu &&
+                           eo_linear_takes(params->eqn, params->order, mesh->K)
+                     : params->order <= EO_MAX_ORDER && params->algorithm != APL_ALGO_CUBATURE_MFMA);
   h->K = mesh->K;
   h->M = M;
   h->Nv = mesh->Nv;
@@ -930,7 +1001,8 @@ int apl_create(const apl_mesh *mesh, const apl_params *params, apl_handle **out)
   if ((rc = dev_upload<int>(h, &h->d_fcode, h->fcode.data(), h->fcode.size()))) return bail(rc);
   if ((rc = dev_upload<int>(h, &h->d_fmask, o.fmask.data(), o.fmask.size()))) return bail(rc);
   if ((rc = dev_upload<double>(h, &h->d_I1D, I1D.data(), I1D.size()))) return bail(rc);
-  if (params->precision == APL_PREC_FP64) rc = upload_fragments<double>(h);
+  if (h->linear && h->eo) rc = upload_eo_linear(h);
+  else if (params->precision == APL_PREC_FP64) rc = upload_fragments<double>(h);
   else if (params->precision == APL_PREC_FP32_MFMA) rc = upload_fragments<float>(h);
   else rc = upload_fragments_bf16x3(h);
   if (rc) return bail(rc);

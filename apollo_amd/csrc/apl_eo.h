@@ -164,9 +164,9 @@ __device__ __forceinline__ void to_vars(const double (&q)[M], double (&x)[MH], d
 // stage (mode 1) or the SSP combination (mode 2), as write_batch does for 16
 // elements.  KEEP: qv holds the group's states as they were staged, and the
 // second operand rb was requested then; else both are read here.
-template <int ES, int NT, bool KEEP>
+template <int ES, int NT, bool KEEP, int EL = 32>
 struct EoOut {
-  static constexpr int NV2 = 32 * ES / 2, NIT = (NV2 + NT - 1) / NT;
+  static constexpr int NV2 = EL * ES / 2, NIT = (NV2 + NT - 1) / NT;
   static __device__ __forceinline__ bool second(const RhsArgs &a) {
     return a.mode == 1 ? a.rk_a != 0.0 : (a.mode == 2 && a.z != nullptr);
   }
@@ -181,7 +181,7 @@ struct EoOut {
                                                    int tid, dbl2 (&qv)[NIT], dbl2 (&rb)[NIT]) {
     const long base = e0 * ES;
     unsigned ef = 0;
-    if (cnt == 32) {
+    if (cnt == EL) {
       const bool two = second(a);
       // one path per mode, so that no select splits the stores
       if (a.mode == 0) {

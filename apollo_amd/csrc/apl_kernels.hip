@@ -5,6 +5,7 @@
 #include "apl_adjoint.h"
 #include "apl_device.h"
 #include "apl_eo.h"
+#include "apl_eo_linear.h"
 #include "apl_limiter.h"
 #include "apl_valu.h"
 
@@ -41,12 +42,45 @@ static int launch_eo(hipStream_t s, const RhsArgs &a) {
   return hipGetLastError() == hipSuccess ? APL_OK : APL_ERR_HIP;
 }
 
+// The even-odd nodal kernel: groups of 64 / EO_LPE elements, W waves each.
+template <int N, int EQN, int FLUX, int W>
+static int launch_eo_linear(hipStream_t s, const RhsArgs &a) {
+  using C = EoLinCfg<N, EQN, W>;
+  auto kern = rhs_eo_linear_kernel<N, EQN, FLUX, W>;
+  const size_t lds = sizeof(double) * (size_t)C::LDS;
+  if (!allow_lds(kern, lds)) return APL_ERR_UNSUPPORTED;
+  hipLaunchKernelGGL(kern, dim3((a.K + C::EL - 1) / C::EL), dim3(64 * W), lds, s, a);
+  return hipGetLastError() == hipSuccess ? APL_OK : APL_ERR_HIP;
+}
+
 // kind: 0 the cubature form on MFMA, 1 the nodal form (linear fluxes) on
 // MFMA, 2 the cubature form on the VALU kernel (N <= 3, FP32), 3 the nodal
 // form on the VALU kernel (TM, FP64 and FP32), 4 the cubature form on the
-// even-odd kernel (N <= 4, FP64)
+// even-odd kernel (N <= 4, FP64), 5 the nodal form on the even-odd kernel
+// (FP64)
 template <int N, int EQN, int FLUX, typename T>
 static int launch_typed(int kind, hipStream_t s, const RhsArgs &a, int nblocks) {
+  if constexpr ((EQN == APL_EQN_PHMAXWELL8 || EQN == APL_EQN_MAXWELL_TM3) && sizeof(T) == 8) {
+    if (kind == 5) {
+      // Four waves per group while a CU's LDS holds its share of the groups,
+      // at most two (us per stage, 4 / 2 waves: 8-variable N = 4, K = 5000,
+      // 14.5 / 17.7; K = 9800, 20.6 / 19.5); then two.  At N <= 4 one, without
+      // the reduction, from four groups per CU on (N = 4: K = 16200 24.5 / 29.5
+      // with one, K = 28800 38.9 / 35.1, K = 180000 212 / 188; N = 5, where one
+      // wave leaves no room for a second one's registers, 241 / 261).
+      const int groups = (a.K + 15) / 16;
+      constexpr int fit = 163840 / (EoLinCfg<N, EQN, 4>::LDS * 8);
+      if constexpr (EQN == APL_EQN_MAXWELL_TM3) {
+        return launch_eo_linear<N, EQN, FLUX, 4>(s, a);
+      } else {
+        if constexpr (fit > 0)
+          if (groups <= 256 * (fit < 2 ? fit : 2)) return launch_eo_linear<N, EQN, FLUX, 4>(s, a);
+        if constexpr (N <= 4)
+          if (groups > 1024) return launch_eo_linear<N, EQN, FLUX, 1>(s, a);
+        return launch_eo_linear<N, EQN, FLUX, 2>(s, a);
+      }
+    }
+  }
   if constexpr (EQN == APL_EQN_PHMAXWELL8 || EQN == APL_EQN_MAXWELL_TM3) {
     if (kind == 1)
       return launch_batches<LinLds<N, EQN, T>::doubles, LinGroup<N, EQN, T>::W>(

@@ -90,7 +90,10 @@ enum apl_algorithm {
                               linear fluxes (Maxwell) the algebraically
                               identical nodal form V V^T Dr_c^T W V_c Q ... on
                               straight-sided elements (no reference
-                              counterpart; same result to rounding).  The
+                              counterpart; same result to rounding), in FP64
+                              by the mirror symmetry of the triangle for the
+                              8-variable system and for TM meshes of at most
+                              8192 elements (4096 at N = 8), else on MFMA.  The
                               cubature form runs on the vector ALU at N <= 4
                               in FP64 and N <= 3 in FP32, on MFMA otherwise  */
   APL_ALGO_CUBATURE = 1,   /* always Apollo's over-integrated cubature form
