@@ -296,7 +296,7 @@ __global__ void __launch_bounds__(64 * W, (AdjEoWaves<N, EQN, W>::value))
 #pragma unroll
       for (int j = 0; j < NIT; ++j) {
         const int idx = tid + NT * j;
-        if (idx < NV2) {
+        if (NT * (j + 1) <= NV2 || idx < NV2) {
           buf[j] = ((const dbl2 *)qb)[idx];
           lam[j] = ((const dbl2 *)lb)[idx];
           if (STAGE) kv[j] = ((const dbl2 *)kb)[idx];
@@ -305,7 +305,7 @@ __global__ void __launch_bounds__(64 * W, (AdjEoWaves<N, EQN, W>::value))
 #pragma unroll
       for (int j = 0; j < NIT; ++j) {
         const int idx = tid + NT * j;
-        if (idx < NV2) {
+        if (NT * (j + 1) <= NV2 || idx < NV2) {
           if (STAGE) lam[j] = lam[j] + a.rk_b * kv[j];
 #pragma unroll
           for (int k = 0; k < 2; ++k) {
@@ -639,13 +639,13 @@ __global__ void __launch_bounds__(64 * W, (AdjEoWaves<N, EQN, W>::value))
 #pragma unroll
       for (int j = 0; j < NIT; ++j) {
         const int idx = tid + NT * j;
-        if (idx < NV2) kv[j] = ((const dbl2 *)(a.qbar + base))[idx];
+        if (NT * (j + 1) <= NV2 || idx < NV2) kv[j] = ((const dbl2 *)(a.qbar + base))[idx];
       }
     }
 #pragma unroll
     for (int j = 0; j < NIT; ++j) {
       const int idx = tid + NT * j;
-      if (idx < NV2) {
+      if (NT * (j + 1) <= NV2 || idx < NV2) {
         const dbl2 v = dbl2{QS[2 * idx], QS[2 * idx + 1]};
         if (v[0] != v[0] || v[1] != v[1]) ef |= EF_NAN;
         if constexpr (!STAGE) {
@@ -694,7 +694,7 @@ __global__ void __launch_bounds__(64 * W, (AdjEoWaves<N, EQN, W>::value))
 #pragma unroll
         for (int j = 0; j < NIT; ++j) {
           const int idx = tid + NT * j;
-          if (idx < NV2) ((dbl2 *)(a.sbar_out + base))[idx] = dbl2{QS[2 * idx], QS[2 * idx + 1]};
+          if (NT * (j + 1) <= NV2 || idx < NV2) ((dbl2 *)(a.sbar_out + base))[idx] = dbl2{QS[2 * idx], QS[2 * idx + 1]};
         }
       } else {
         for (int i = tid; i < cnt * ES; i += NT) a.sbar_out[base + i] = QS[i];

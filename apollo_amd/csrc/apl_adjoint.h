@@ -229,7 +229,7 @@ __device__ __forceinline__ void axpy_stage_transposed(double *XT, const double *
 #pragma unroll
     for (int j = 0; j < NIT; ++j) {
       const int idx = lane + 64 * j;
-      if (idx < NV2) {
+      if (64 * (j + 1) <= NV2 || idx < NV2) {
         yv[j] = ((const dbl2 *)y)[idx];
         xv[j] = ((const dbl2 *)x)[idx];
       }
@@ -237,7 +237,7 @@ __device__ __forceinline__ void axpy_stage_transposed(double *XT, const double *
 #pragma unroll
     for (int j = 0; j < NIT; ++j) {
       const int idx = lane + 64 * j;
-      if (idx < NV2) {
+      if (64 * (j + 1) <= NV2 || idx < NV2) {
         const dbl2 v = yv[j] + b * xv[j];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -266,7 +266,7 @@ __device__ __forceinline__ void copy_batch(double *dst, const double *src, int c
 #pragma unroll
     for (int j = 0; j < NIT; ++j) {
       const int idx = lane + 64 * j;
-      if (idx < NV2) ((dbl2 *)dst)[idx] = dbl2{src[2 * idx], src[2 * idx + 1]};
+      if (64 * (j + 1) <= NV2 || idx < NV2) ((dbl2 *)dst)[idx] = dbl2{src[2 * idx], src[2 * idx + 1]};
     }
   } else {
     for (int i = lane; i < cnt * ES; i += 64) dst[i] = src[i];
@@ -386,13 +386,13 @@ __device__ __forceinline__ unsigned adj_write_batch(const AdjArgs &a, const doub
 #pragma unroll
       for (int j = 0; j < NIT; ++j) {
         const int idx = lane + 64 * j;
-        if (idx < NV2) qv[j] = ((const dbl2 *)(a.qbar + base))[idx];
+        if (64 * (j + 1) <= NV2 || idx < NV2) qv[j] = ((const dbl2 *)(a.qbar + base))[idx];
       }
     }
 #pragma unroll
     for (int j = 0; j < NIT; ++j) {
       const int idx = lane + 64 * j;
-      if (idx < NV2) {
+      if (64 * (j + 1) <= NV2 || idx < NV2) {
         const dbl2 v = dbl2{OUT[2 * idx], OUT[2 * idx + 1]};
         if (v[0] != v[0] || v[1] != v[1]) ef |= EF_NAN;
         if constexpr (!STAGE) {

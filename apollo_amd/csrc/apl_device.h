@@ -735,7 +735,12 @@ typedef double dbl2 __attribute__((ext_vector_type(2)));
 
 // XT[w*RS + e] = q[(e0 + e)*ES + w]: all loads of a full batch are issued
 // before any LDS write (16-byte vector loads; the batch base is 128-byte
-// aligned because 16*ES*8 is a multiple of 128).
+// aligned because 16*ES*8 is a multiple of 128).  Only the last of the NIT
+// loads can lie past the batch; the others carry no bound check, for as
+// branches the checks split the loads and keep values live across them (us
+// per stage without / with, FP64: TM N = 5, K = 131072 68.0 / 70.5; Euler
+// N = 5, K = 131072 293 / 327; BF16x3 Euler N = 4, K = 181202 150 / 156; in
+// the even-odd kernels' copies Euler N = 4, K = 524288 401 / 411).
 template <int ES, int RS = XS, typename XE = double>
 __device__ __forceinline__ void stage_transposed(XE *XT, const double *qb, int cnt, int lane) {
   constexpr int NV2 = 16 * ES / 2;
@@ -745,12 +750,12 @@ __device__ __forceinline__ void stage_transposed(XE *XT, const double *qb, int c
 #pragma unroll
     for (int j = 0; j < NIT; ++j) {
       const int idx = lane + 64 * j;
-      if (idx < NV2) buf[j] = ((const dbl2 *)qb)[idx];
+      if (64 * (j + 1) <= NV2 || idx < NV2) buf[j] = ((const dbl2 *)qb)[idx];
     }
 #pragma unroll
     for (int j = 0; j < NIT; ++j) {
       const int idx = lane + 64 * j;
-      if (idx < NV2) {
+      if (64 * (j + 1) <= NV2 || idx < NV2) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const int i = 2 * idx + h, e = i / ES, w = i - e * ES;
@@ -783,7 +788,7 @@ __device__ __forceinline__ unsigned write_batch(const RhsArgs &a, const OE *OUT,
 #pragma unroll
       for (int j = 0; j < NIT; ++j) {
         const int idx = lane + 64 * j;
-        if (idx < NV2) {
+        if (64 * (j + 1) <= NV2 || idx < NV2) {
           qv[j] = ((const dbl2 *)(a.q + base))[idx];
           if (a.z) zv[j] = ((const dbl2 *)(a.z + base))[idx];
         }
@@ -791,7 +796,7 @@ __device__ __forceinline__ unsigned write_batch(const RhsArgs &a, const OE *OUT,
 #pragma unroll
       for (int j = 0; j < NIT; ++j) {
         const int idx = lane + 64 * j;
-        if (idx < NV2) {
+        if (64 * (j + 1) <= NV2 || idx < NV2) {
           const dbl2 v = dbl2{OUT[2 * idx], OUT[2 * idx + 1]};
           if (v[0] != v[0] || v[1] != v[1]) ef |= EF_NAN;
           dbl2 o = a.ca * qv[j] + a.cb * v;
@@ -815,7 +820,7 @@ __device__ __forceinline__ unsigned write_batch(const RhsArgs &a, const OE *OUT,
 #pragma unroll
       for (int j = 0; j < NIT; ++j) {
         const int idx = lane + 64 * j;
-        if (idx < NV2) {
+        if (64 * (j + 1) <= NV2 || idx < NV2) {
           const dbl2 v = dbl2{OUT[2 * idx], OUT[2 * idx + 1]};
           if (v[0] != v[0] || v[1] != v[1]) ef |= EF_NAN;
           ((dbl2 *)(a.out + base))[idx] = v;
@@ -826,7 +831,7 @@ __device__ __forceinline__ unsigned write_batch(const RhsArgs &a, const OE *OUT,
 #pragma unroll
       for (int j = 0; j < NIT; ++j) {
         const int idx = lane + 64 * j;
-        if (idx < NV2) {
+        if (64 * (j + 1) <= NV2 || idx < NV2) {
           if (a.rk_a != 0.0) rb[j] = ((const dbl2 *)(a.res + base))[idx];
           qv[j] = ((const dbl2 *)(a.q + base))[idx];
         }
@@ -834,7 +839,7 @@ __device__ __forceinline__ unsigned write_batch(const RhsArgs &a, const OE *OUT,
 #pragma unroll
       for (int j = 0; j < NIT; ++j) {
         const int idx = lane + 64 * j;
-        if (idx < NV2) {
+        if (64 * (j + 1) <= NV2 || idx < NV2) {
           dbl2 r;
 #pragma unroll
           for (int h = 0; h < 2; ++h) {

@@ -174,7 +174,7 @@ struct EoOut {
 #pragma unroll
     for (int j = 0; j < NIT; ++j) {
       const int idx = tid + NT * j;
-      if (idx < NV2) v[j] = ((const dbl2 *)(p + base))[idx];
+      if (NT * (j + 1) <= NV2 || idx < NV2) v[j] = ((const dbl2 *)(p + base))[idx];
     }
   }
   static __device__ __forceinline__ unsigned write(const RhsArgs &a, const double *OUT, long e0, int cnt,
@@ -188,7 +188,7 @@ struct EoOut {
 #pragma unroll
         for (int j = 0; j < NIT; ++j) {
           const int idx = tid + NT * j;
-          if (idx < NV2) {
+          if (NT * (j + 1) <= NV2 || idx < NV2) {
             const dbl2 v = dbl2{OUT[2 * idx], OUT[2 * idx + 1]};
             if (v[0] != v[0] || v[1] != v[1]) ef |= EF_NAN;
             ((dbl2 *)(a.out + base))[idx] = v;
@@ -203,7 +203,7 @@ struct EoOut {
 #pragma unroll
         for (int j = 0; j < NIT; ++j) {
           const int idx = tid + NT * j;
-          if (idx < NV2) {
+          if (NT * (j + 1) <= NV2 || idx < NV2) {
             const dbl2 v = dbl2{OUT[2 * idx], OUT[2 * idx + 1]};
             if (v[0] != v[0] || v[1] != v[1]) ef |= EF_NAN;
             const dbl2 r = two ? a.rk_a * (KEEP ? rb[j] : r1[j]) + a.dt * v : a.dt * v;
@@ -220,7 +220,7 @@ struct EoOut {
 #pragma unroll
         for (int j = 0; j < NIT; ++j) {
           const int idx = tid + NT * j;
-          if (idx < NV2) {
+          if (NT * (j + 1) <= NV2 || idx < NV2) {
             const dbl2 v = dbl2{OUT[2 * idx], OUT[2 * idx + 1]};
             if (v[0] != v[0] || v[1] != v[1]) ef |= EF_NAN;
             dbl2 o = a.ca * (KEEP ? qv[j] : q1[j]) + a.cb * v;
@@ -332,7 +332,7 @@ __global__ void __launch_bounds__(64 * W, (EoWaves<N, EQN, W>::value))
 #pragma unroll
       for (int j = 0; j < NIT; ++j) {
         const int idx = tid + NT * j;
-        if (idx < NV2) {
+        if (NT * (j + 1) <= NV2 || idx < NV2) {
 #pragma unroll
           for (int k = 0; k < 2; ++k) {
             const int i = 2 * idx + k, e = i / ES, w = i - e * ES;

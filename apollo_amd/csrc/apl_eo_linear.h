@@ -233,7 +233,7 @@ __global__ void __launch_bounds__(64 * W, (EoLinWaves<N, EQN>::value))
 #pragma unroll
       for (int j = 0; j < NIT; ++j) {
         const int idx = tid + NT * j;
-        if (idx < NV2) {
+        if (NT * (j + 1) <= NV2 || idx < NV2) {
 #pragma unroll
           for (int k = 0; k < 2; ++k) {
             const int i = 2 * idx + k, e = i / ES, w = i - e * ES;
@@ -394,7 +394,6 @@ __global__ void __launch_bounds__(64 * W, (EoLinWaves<N, EQN>::value))
   }
 
   // 5. the stage update and the store; every element sees the same speed
-  __builtin_amdgcn_sched_barrier(0);   // its loads stay below the residual's last use
   dbl2 none[NIT];
   ef |= Out::write(a, QS, e0, cnt, tid, none, none);
   for (int off = 32; off > 0; off >>= 1) ef |= __shfl_xor(ef, off);

@@ -138,12 +138,12 @@ __global__ void __launch_bounds__(64 * W, VALU_WAVES)
 #pragma unroll
       for (int j = 0; j < NIT; ++j) {
         const int idx = tid + NT * j;
-        if (idx < NV2) buf[j] = ((const dbl2 *)qb)[idx];
+        if (NT * (j + 1) <= NV2 || idx < NV2) buf[j] = ((const dbl2 *)qb)[idx];
       }
 #pragma unroll
       for (int j = 0; j < NIT; ++j) {
         const int idx = tid + NT * j;
-        if (idx < NV2) {
+        if (NT * (j + 1) <= NV2 || idx < NV2) {
 #pragma unroll
           for (int h = 0; h < 2; ++h) {
             const int i = 2 * idx + h, e = i / ES, w = i - e * ES;
@@ -468,12 +468,12 @@ __global__ void __launch_bounds__((64 * ValuLinCfg<N, EQN>::W), (ValuLinWaves<N,
 #pragma unroll
       for (int j = 0; j < NIT; ++j) {
         const int idx = tid + NT * j;
-        if (idx < NV2) buf[j] = ((const dbl2 *)qb)[idx];
+        if (NT * (j + 1) <= NV2 || idx < NV2) buf[j] = ((const dbl2 *)qb)[idx];
       }
 #pragma unroll
       for (int j = 0; j < NIT; ++j) {
         const int idx = tid + NT * j;
-        if (idx < NV2) {
+        if (NT * (j + 1) <= NV2 || idx < NV2) {
 #pragma unroll
           for (int h = 0; h < 2; ++h) {
             const int i = 2 * idx + h, e = i / ES, w = i - e * ES;
