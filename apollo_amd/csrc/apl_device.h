@@ -731,6 +731,23 @@ __device__ __forceinline__ WaveBatch wave_batch(int K) {
   return w;
 }
 
+// Node numbering: row j (j = 0..N) holds nodes (i, j), i = 0..N-j; the mirror
+// of the reference triangle swaps i and j.
+constexpr int eo_node(int N, int i, int j) { return j * (N + 1) - j * (j - 1) / 2 + i; }
+
+// Face node i of face f: bottom left to right, hypotenuse upwards, left side
+// downwards (the reference's Fmask; checked against it at creation).
+constexpr int eo_fmask(int N, int f, int i) {
+  return f == 0 ? eo_node(N, i, 0) : (f == 1 ? eo_node(N, N - i, i) : eo_node(N, 0, N - i));
+}
+
+// The same without branches, for a lane's own f and i.
+template <int N>
+__device__ __forceinline__ int face_node(int f, int i) {
+  const int row = f == 0 ? 0 : (f == 1 ? i : N - i), col = f == 0 ? i : (f == 1 ? N - i : 0);
+  return row * (2 * N + 3 - row) / 2 + col;
+}
+
 typedef double dbl2 __attribute__((ext_vector_type(2)));
 
 // XT[w*RS + e] = q[(e0 + e)*ES + w]: all loads of a full batch are issued
@@ -741,25 +758,36 @@ typedef double dbl2 __attribute__((ext_vector_type(2)));
 // per stage without / with, FP64: TM N = 5, K = 131072 68.0 / 70.5; Euler
 // N = 5, K = 131072 293 / 327; BF16x3 Euler N = 4, K = 181202 150 / 156; in
 // the even-odd kernels' copies Euler N = 4, K = 524288 401 / 411).
-template <int ES, int RS = XS, typename XE = double>
-__device__ __forceinline__ void stage_transposed(XE *XT, const double *qb, int cnt, int lane) {
-  constexpr int NV2 = 16 * ES / 2;
-  constexpr int NIT = (NV2 + 63) / 64;
+template <int ES>
+struct StageBuf {
+  static constexpr int NV2 = 16 * ES / 2, NIT = (NV2 + 63) / 64;
+  dbl2 v[NIT];
+};
+
+template <int ES>
+__device__ __forceinline__ void stage_load(StageBuf<ES> &buf, const double *qb, int cnt, int lane) {
+  using B = StageBuf<ES>;
   if (cnt == 16) {
-    dbl2 buf[NIT];
 #pragma unroll
-    for (int j = 0; j < NIT; ++j) {
+    for (int j = 0; j < B::NIT; ++j) {
       const int idx = lane + 64 * j;
-      if (64 * (j + 1) <= NV2 || idx < NV2) buf[j] = ((const dbl2 *)qb)[idx];
+      if (64 * (j + 1) <= B::NV2 || idx < B::NV2) buf.v[j] = ((const dbl2 *)qb)[idx];
     }
+  }
+}
+
+template <int ES, int RS = XS, typename XE = double>
+__device__ __forceinline__ void stage_store(XE *XT, const StageBuf<ES> &buf, const double *qb, int cnt, int lane) {
+  using B = StageBuf<ES>;
+  if (cnt == 16) {
 #pragma unroll
-    for (int j = 0; j < NIT; ++j) {
+    for (int j = 0; j < B::NIT; ++j) {
       const int idx = lane + 64 * j;
-      if (64 * (j + 1) <= NV2 || idx < NV2) {
+      if (64 * (j + 1) <= B::NV2 || idx < B::NV2) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const int i = 2 * idx + h, e = i / ES, w = i - e * ES;
-          XT[w * RS + e] = XE(buf[j][h]);
+          XT[w * RS + e] = XE(buf.v[j][h]);
         }
       }
     }
@@ -769,6 +797,13 @@ __device__ __forceinline__ void stage_transposed(XE *XT, const double *qb, int c
       XT[w * RS + e] = XE((e < cnt) ? qb[i] : qb[w]);
     }
   }
+}
+
+template <int ES, int RS = XS, typename XE = double>
+__device__ __forceinline__ void stage_transposed(XE *XT, const double *qb, int cnt, int lane) {
+  StageBuf<ES> buf;
+  stage_load<ES>(buf, qb, cnt, lane);
+  stage_store<ES, RS, XE>(XT, buf, qb, cnt, lane);
 }
 
 // Write the batch result OUT[e*ES + w] (LDS): rhs (mode 0), the LSERK4
@@ -1420,24 +1455,22 @@ struct LinOrder {
   static constexpr int NKP = (3 * Order<N>::Nfp + 3) / 4;   // k-steps of the face GEMM
 };
 
-// The neighbour's values at face node kf = f Nfp + i of an element (its
-// node Fmask[nf][Nfp-1-i], given as fnb[nf]); zero on boundary faces and
-// past the last face node.
-template <int Np, int Nfp, int M>
+// The neighbour's values at face node kf = f Nfp + i of element ge (its
+// node Fmask[nf][Nfp-1-i]); the element's own values there on boundary faces
+// (boundary_state sets them), of face 0 past the last face node.  Branch-free:
+// as branches, with the node numbers read from a table, each node's loads
+// waited for the table entry that its branch read, and with it for every load
+// before it.
+template <int N, int M>
 __device__ __forceinline__ void gather_face_node(const double *q, int kf, int code0, int code1,
-                                                 int code2, const int (&fnb)[3], double *dst) {
-  const int f = kf / Nfp;
+                                                 int code2, long ge, double *dst) {
+  constexpr int Np = Order<N>::Np, Nfp = N + 1;
+  const int f = kf < 3 * Nfp ? kf / Nfp : 0, i = kf < 3 * Nfp ? kf - f * Nfp : 0;
   const int code = f == 0 ? code0 : (f == 1 ? code1 : code2);
-  if (kf < 3 * Nfp && code >= 0) {
-    const int nf = code & 3;
-    const int node = nf == 0 ? fnb[0] : (nf == 1 ? fnb[1] : fnb[2]);
-    const double *src = q + ((long)(code >> 2) * Np + node) * M;
+  const double *src = q + ((code >= 0 ? (long)(code >> 2) : ge) * Np +
+                           face_node<N>(code >= 0 ? code & 3 : 0, Nfp - 1 - i)) * M;
 #pragma unroll
-    for (int v = 0; v < M; ++v) dst[v] = src[v];
-  } else {
-#pragma unroll
-    for (int v = 0; v < M; ++v) dst[v] = 0.0;
-  }
+  for (int v = 0; v < M; ++v) dst[v] = src[v];
 }
 
 // Waves per SIMD requested from the register allocator (a lower bound: the
@@ -1497,19 +1530,7 @@ __global__ void __launch_bounds__((64 * LinGroup<N, EQN, T>::W), (LinWaves<N, EQ
   const double *gk = a.geom + ge * G_WORDS;
   const int code0 = a.fcode[ge * 3], code1 = a.fcode[ge * 3 + 1], code2 = a.fcode[ge * 3 + 2];
 
-  // face node kf = 4 j + lg of element el: own node Fmask[f][i] and the
-  // neighbour's node Fmask[nf][Nfp-1-i] for each possible neighbour face nf
-  int fown[NKP], fnb[NKP][3];
-#pragma unroll
-  for (int j = 0; j < NKP; ++j) {
-    const int kf = 4 * j + lg;
-    const int f = kf < 3 * Nfp ? kf / Nfp : 0, i = kf < 3 * Nfp ? kf - f * Nfp : 0;
-    fown[j] = a.fmask[f * Nfp + i];
-#pragma unroll
-    for (int nf = 0; nf < 3; ++nf) fnb[j][nf] = a.fmask[nf * Nfp + (Nfp - 1 - i)];
-  }
-
-  // Neighbour face-node values (zero on boundary faces).  FP32 and BF16x3 up
+  // Neighbour face-node values.  FP32 and BF16x3 up
   // to 5 variables load them all into registers before the batch staging,
   // so their latency overlaps it; FP64 and phMaxwell load them per k-step
   // (FP64, measured: K = 131072, N = 5 80.7 -> 77.5 us per stage;
@@ -1518,13 +1539,22 @@ __global__ void __launch_bounds__((64 * LinGroup<N, EQN, T>::W), (LinWaves<N, EQ
   const double *qg = a.q;
   constexpr bool PRE = M <= 5 && sizeof(T) != 8;
   double qP[PRE ? NKP : 1][M];
+  // The gather's addresses wait for the face codes.  At N >= 7 the state's
+  // loads go out before that wait, below after it (FP32, us per stage, state
+  // first / gather first: N = 8, K = 294912 348 / 356, K = 8192 19.1 / 18.6;
+  // N = 5, K = 8192 12.5 / 12.1, K = 180000 107 / 108).
+  constexpr bool EARLY = N >= 7;
+  StageBuf<ES> buf;
+  if constexpr (EARLY || !PRE) stage_load<ES>(buf, a.q + e0 * ES, cnt, lane);
   if constexpr (PRE) {
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < NKP; ++j)
-      gather_face_node<Np, Nfp, M>(qg, 4 * j + lg, code0, code1, code2, fnb[j], qP[j]);
+      gather_face_node<N, M>(qg, 4 * j + lg, code0, code1, code2, ge, qP[j]);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (!EARLY) stage_load<ES>(buf, a.q + e0 * ES, cnt, lane);
   }
-
-  stage_transposed<ES, XS, XE>(XT, a.q + e0 * ES, cnt, lane);
+  stage_store<ES, XS, XE>(XT, buf, a.q + e0 * ES, cnt, lane);
   for (int i = ES * XS + lane; i < L::XT; i += 64) XT[i] = XE(0);
   wave_sync();
 
@@ -1553,14 +1583,14 @@ __global__ void __launch_bounds__((64 * LinGroup<N, EQN, T>::W), (LinWaves<N, EQ
     }
     S fsT[M];
     if (kf < 3 * Nfp) {
-      const int f = kf / Nfp;
+      const int f = kf / Nfp, own = face_node<N>(f, kf - f * Nfp);
       const int code = f == 0 ? code0 : (f == 1 ? code1 : code2);
       const double nx = gk[G_NX + f], ny = gk[G_NY + f], sj = gk[G_SJ + f];
       double qM[M], fs[M];
       double *qp = qP[PRE ? ks : 0];
-      if constexpr (!PRE) gather_face_node<Np, Nfp, M>(qg, kf, code0, code1, code2, fnb[ks], qp);
+      if constexpr (!PRE) gather_face_node<N, M>(qg, kf, code0, code1, code2, ge, qp);
 #pragma unroll
-      for (int v = 0; v < M; ++v) qM[v] = double(XT[(fown[ks] * M + v) * XS + el]);
+      for (int v = 0; v < M; ++v) qM[v] = double(XT[(own * M + v) * XS + el]);
       if (code < 0) boundary_state<EQN>(*a.bc, -code - 1, 0.0, 0.0, 0.0, nx, ny, qM, qp);
       double lam;
       ef |= num_flux<EQN, FLUX>(a.ph, nx, ny, qM, qp, fs, &lam);

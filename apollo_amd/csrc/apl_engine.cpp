@@ -916,6 +916,12 @@ int apl_create(const apl_mesh *mesh, const apl_params *params, apl_handle **out)
     return bail(APL_ERR_ORDER);
   }
   const Operators &o = h->ops;
+  for (int f = 0; f < 3; ++f)
+    for (int i = 0; i < o.Nfp; ++i)
+      if (o.fmask[f * o.Nfp + i] != eo_fmask(o.N, f, i)) {
+        h->last_error = "the order's face nodes are not numbered as the kernels assume";
+        return bail(APL_ERR_ORDER);
+      }
   int bad = -1;
   int rc = build_geometry(o, h->K, mesh->VX, mesh->VY, mesh->EToV, h->geo, bad);
   if (rc) {

@@ -39,16 +39,6 @@
 
 namespace apl {
 
-// Node numbering: row j (j = 0..N) holds nodes (i, j), i = 0..N-j; the mirror
-// swaps i and j.
-constexpr int eo_node(int N, int i, int j) { return j * (N + 1) - j * (j - 1) / 2 + i; }
-
-// Face node i of face f: bottom left to right, hypotenuse upwards, left side
-// downwards (the reference's Fmask; checked against it at creation).
-constexpr int eo_fmask(int N, int f, int i) {
-  return f == 0 ? eo_node(N, i, 0) : (f == 1 ? eo_node(N, N - i, i) : eo_node(N, 0, N - i));
-}
-
 // cubature points on the mirror axis of the rule of order N (checked at
 // creation against the rule)
 constexpr int eo_axis_points(int N) {

@@ -170,7 +170,7 @@ struct EoFaceNode {
 };
 
 template <int N, int M>
-__device__ __forceinline__ void eo_face_node(const double *q, const int *fmask, const double *gk, int kf,
+__device__ __forceinline__ void eo_face_node(const double *q, const double *gk, int kf,
                                              int code0, int code1, int code2, long ge, EoFaceNode<M> &F) {
   constexpr int Np = Order<N>::Np, Nfp = N + 1;
   const int f = kf / Nfp, i = kf - f * Nfp;
@@ -178,9 +178,9 @@ __device__ __forceinline__ void eo_face_node(const double *q, const int *fmask, 
   F.nx = gk[G_NX + f];
   F.ny = gk[G_NY + f];
   F.sj = gk[G_SJ + f];
-  F.own = fmask[kf] * M;
+  F.own = face_node<N>(f, i) * M;
   const int nf = F.code >= 0 ? (F.code & 3) : 0;
-  const double *src = q + ((F.code >= 0 ? (long)(F.code >> 2) : ge) * Np + fmask[nf * Nfp + (Nfp - 1 - i)]) * M;
+  const double *src = q + ((F.code >= 0 ? (long)(F.code >> 2) : ge) * Np + face_node<N>(nf, Nfp - 1 - i)) * M;
 #pragma unroll
   for (int v = 0; v < M; ++v) F.qP[v] = src[v];
 }
@@ -251,7 +251,7 @@ __global__ void __launch_bounds__(64 * W, (EoLinWaves<N, EQN>::value))
 
   const int fb = max(ub - NVU, 0), fe = max(ue - NVU, 0);
   EoFaceNode<M> F;
-  if (fb < fe) eo_face_node<N, M>(a.q, a.fmask, gk, tab[(NVU + fb) * C::LPE + qd], code0, code1, code2, ge, F);
+  if (fb < fe) eo_face_node<N, M>(a.q, gk, tab[(NVU + fb) * C::LPE + qd], code0, code1, code2, ge, F);
   group_sync<W>();
 
   const double *qe = QS + el * ESP;
@@ -303,7 +303,7 @@ __global__ void __launch_bounds__(64 * W, (EoLinWaves<N, EQN>::value))
   for (int u = fb; u < fe; ++u) {
     const EoFaceNode<M> G = F;
     if (u + 1 < fe)
-      eo_face_node<N, M>(a.q, a.fmask, gk, tab[(NVU + u + 1) * C::LPE + qd], code0, code1, code2, ge, F);
+      eo_face_node<N, M>(a.q, gk, tab[(NVU + u + 1) * C::LPE + qd], code0, code1, code2, ge, F);
     double qM[M], qP[M], f[M], y[LPE][MH];
 #pragma unroll
     for (int v = 0; v < M; ++v) {
