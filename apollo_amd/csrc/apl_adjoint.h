@@ -39,7 +39,6 @@ struct AdjArgs {
   const double *vert;
   const int *fcode;
   const double *I1D;        // [3][Ng][Nfp] + Gauss abscissae
-  const int *fmask;
   const double *Avc;        // V_c fragments        [NCH][NKS1][64]
   const double *Aart;       // A_r^T fragments      [NCH][NKS1][64]
   const double *Aast;       // A_s^T fragments      [NCH][NKS1][64]
@@ -447,7 +446,7 @@ struct AdjLds {
   static constexpr int XT = Order<N>::NKS1 * 4 * M * 16;
   static constexpr int PT = 3 * Nfp * M * 16;
   static constexpr int I1D = 3 * Ng * Nfp;
-  static constexpr int MAIN = 2 * XT + PT + I1D + 2 * Nfp;
+  static constexpr int MAIN = 2 * XT + PT + I1D;
   // epilogue: OUT (16 ES, inside XT's space), then SO (16 FS) over it; the
   // staged lam (LT) is read while the next lam is staged past both
   static constexpr int SO = 16 * 3 * Ng * M > 2 * XT ? 16 * 3 * Ng * M : 2 * XT;
@@ -493,7 +492,6 @@ __global__ void __launch_bounds__((64 * AdjGroup<N, EQN>::W), (AdjWaves<N, EQN>:
   double *LT = XT + L::XT;          // lam / J, transposed
   double *PT = LT + L::XT;          // neighbour face nodes (own order)
   double *I1 = PT + L::PT;
-  int *FM = (int *)(I1 + L::I1D);
 
   const int lane = wb.lane, el = lane & 15, lg = lane >> 4;
   const long e0 = wb.e0;
@@ -504,25 +502,35 @@ __global__ void __launch_bounds__((64 * AdjGroup<N, EQN>::W), (AdjWaves<N, EQN>:
 
   // 1/J of lane el's element (0 past the batch end) scales the lam operands
   const double sc = el < cnt ? gk[G_INVJ] : 0.0;
-  for (int i = lane; i < L::I1D; i += 64) I1[i] = a.I1D[i];
-  for (int i = lane; i < 3 * Nfp; i += 64) FM[i] = a.fmask[i];
-  stage_transposed<ES, 16>(XT, a.q + e0 * ES, cnt, lane);
+  // the tables, the neighbours' face nodes and the state requested at once
+  // (as in rhs_kernel)
+  const int code0 = a.fcode[ge * 3], code1 = a.fcode[ge * 3 + 1], code2 = a.fcode[ge * 3 + 2];
+  constexpr int NGI = (3 * Nfp + 3) / 4, NI1 = (L::I1D + 63) / 64;
+  double i1v[NI1], nbv[NGI][M];
+#pragma unroll
+  for (int j = 0; j < NI1; ++j) i1v[j] = a.I1D[min(lane + 64 * j, L::I1D - 1)];
+  StageBuf<ES> buf;
+  stage_load<ES>(buf, a.q + e0 * ES, cnt, lane);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int j = 0; j < NGI; ++j)
+    gather_face_node<N, M>(a.q, 4 * j + lg, code0, code1, code2, ge, nbv[j]);
+  __builtin_amdgcn_sched_barrier(0);
+  stage_store<ES, 16>(XT, buf, a.q + e0 * ES, cnt, lane);
   if constexpr (STAGE)
     axpy_stage_transposed<ES>(LT, a.lam + e0 * ES, a.qbar + e0 * ES, a.rk_b, cnt, lane);
   else
     stage_transposed<ES, 16>(LT, a.lam + e0 * ES, cnt, lane);
   for (int i = 16 * ES + lane; i < L::XT; i += 64) XT[i] = LT[i] = 0.0;
-  wave_sync();
-  for (int it = lane; it < 16 * 3 * Nfp; it += 64) {
-    const int e = it & 15, k = it >> 4, f = k / Nfp, i = k - f * Nfp;
-    const long gee = e0 + (e < cnt ? e : 0);
-    const int code = a.fcode[gee * 3 + f];
 #pragma unroll
-    for (int v = 0; v < M; ++v) {
-      double pv = 0.0;
-      if (code >= 0)
-        pv = a.q[((long)(code >> 2) * Np + FM[(code & 3) * Nfp + (Nfp - 1 - i)]) * M + v];
-      PT[(k * M + v) * 16 + e] = pv;
+  for (int j = 0; j < NI1; ++j)
+    if (64 * (j + 1) <= L::I1D || lane + 64 * j < L::I1D) I1[lane + 64 * j] = i1v[j];
+#pragma unroll
+  for (int j = 0; j < NGI; ++j) {
+    const int k = 4 * j + lg;
+    if (4 * j + 4 <= 3 * Nfp || k < 3 * Nfp) {
+#pragma unroll
+      for (int v = 0; v < M; ++v) PT[(k * M + v) * 16 + el] = nbv[j][v];
     }
   }
   wave_sync();
@@ -586,7 +594,6 @@ __global__ void __launch_bounds__((64 * AdjGroup<N, EQN>::W), (AdjWaves<N, EQN>:
   }
 
   // surface
-  const int code0 = a.fcode[ge * 3], code1 = a.fcode[ge * 3 + 1], code2 = a.fcode[ge * 3 + 2];
   unsigned ef = 0;
 #pragma unroll 1
   for (int ks = 0; ks < NKF; ++ks) {
@@ -604,7 +611,7 @@ __global__ void __launch_bounds__((64 * AdjGroup<N, EQN>::W), (AdjWaves<N, EQN>:
       const double *Io = I1 + (f * Ng + g) * Nfp;
 #pragma unroll
       for (int i = 0; i < Nfp; ++i) {
-        const double *xo = XT + FM[f * Nfp + i] * M * 16 + el;
+        const double *xo = XT + face_node_at<N>(f, i) * M * 16 + el;
 #pragma unroll
         for (int v = 0; v < M; ++v) qM[v] += Io[i] * xo[v * 16];
       }

@@ -748,6 +748,12 @@ __device__ __forceinline__ int face_node(int f, int i) {
   return row * (2 * N + 3 - row) / 2 + col;
 }
 
+// Of a lane's own f and an i known at compile time.
+template <int N>
+__device__ __forceinline__ int face_node_at(int f, int i) {
+  return f == 0 ? eo_fmask(N, 0, i) : (f == 1 ? eo_fmask(N, 1, i) : eo_fmask(N, 2, i));
+}
+
 typedef double dbl2 __attribute__((ext_vector_type(2)));
 
 // XT[w*RS + e] = q[(e0 + e)*ES + w]: all loads of a full batch are issued
@@ -901,6 +907,24 @@ __device__ __forceinline__ unsigned write_batch(const RhsArgs &a, const OE *OUT,
     }
   }
   return ef;
+}
+
+// The neighbour's values at face node kf = f Nfp + i of element ge (its
+// node Fmask[nf][Nfp-1-i]); the element's own values there on boundary faces
+// (boundary_state sets them), of face 0 past the last face node.  Branch-free:
+// as branches, with the node numbers read from a table, each node's loads
+// waited for the table entry that its branch read, and with it for every load
+// before it.
+template <int N, int M>
+__device__ __forceinline__ void gather_face_node(const double *q, int kf, int code0, int code1,
+                                                 int code2, long ge, double *dst) {
+  constexpr int Np = Order<N>::Np, Nfp = N + 1;
+  const int f = kf < 3 * Nfp ? kf / Nfp : 0, i = kf < 3 * Nfp ? kf - f * Nfp : 0;
+  const int code = f == 0 ? code0 : (f == 1 ? code1 : code2);
+  const double *src = q + ((code >= 0 ? (long)(code >> 2) : ge) * Np +
+                           face_node<N>(code >= 0 ? code & 3 : 0, Nfp - 1 - i)) * M;
+#pragma unroll
+  for (int v = 0; v < M; ++v) dst[v] = src[v];
 }
 
 // ---------------------------------------------------------------------------
@@ -1165,37 +1189,42 @@ __global__ void __launch_bounds__((64 * RhsGroup<N, EQN, T>::W), (MinWaves<N, EQ
   const double sj0 = gk[G_SJ], sj1 = gk[G_SJ + 1], sj2 = gk[G_SJ + 2];
   const int code0 = a.fcode[ge * 3], code1 = a.fcode[ge * 3 + 1], code2 = a.fcode[ge * 3 + 2];
 
-  // 1. small tables
-  for (int i = lane; i < L::I1D; i += 64) I1[i] = a.I1D[i];
-  for (int i = lane; i < 3 * Nfp; i += 64) FM[i] = a.fmask[i];
+  // 1. everything the wave reads before its first product, requested at once:
+  // the small tables, the batch state (coalesced), the neighbours' face nodes
+  // (item k = f Nfp + i of the lane's element, 4 j + lg; their addresses wait
+  // for the face codes, so they go last: FP64 N = 5, K = 80000 170 us per
+  // stage, before the state 181).  As dependent loops -- table, state, then per
+  // item the code, the node number and the values -- this took ten latencies
+  // (us per stage, before -> after: BF16x3 Euler N = 4, K = 181202 150 -> 135,
+  // K = 1152 20.3 -> 19.0; FP32 N = 5, K = 80000 104 -> 91; FP64 N = 5 183 ->
+  // 168).
+  constexpr int NGI = (3 * Nfp + 3) / 4, NI1 = (L::I1D + 63) / 64;
+  double i1v[NI1];
+#pragma unroll
+  for (int j = 0; j < NI1; ++j) i1v[j] = a.I1D[min(lane + 64 * j, L::I1D - 1)];
+  const int fmv = a.fmask[min(lane, 3 * Nfp - 1)];
+  StageBuf<ES> buf;
+  stage_load<ES>(buf, a.q + e0 * ES, cnt, lane);
+  __builtin_amdgcn_sched_barrier(0);
+  double nbv[NGI][M];
+#pragma unroll
+  for (int j = 0; j < NGI; ++j)
+    gather_face_node<N, M>(a.q, 4 * j + lg, code0, code1, code2, ge, nbv[j]);
+  __builtin_amdgcn_sched_barrier(0);
 
-  // 2. stage the batch state, transposed (coalesced global reads)
-  stage_transposed<ES, XS, XE>(XT, a.q + e0 * ES, cnt, lane);
+  // 2. to LDS: the state transposed, the tables, the neighbours' values
+  stage_store<ES, XS, XE>(XT, buf, a.q + e0 * ES, cnt, lane);
   for (int i = ES * XS + lane; i < L::XT; i += 64) XT[i] = XE(0);
-  wave_sync();
-
-  // 3. gather the neighbours' face nodes; item (k = f*Nfp + i, e), e fastest
-  constexpr int NGI = (16 * 3 * Nfp + 63) / 64;
+#pragma unroll
+  for (int j = 0; j < NI1; ++j)
+    if (64 * (j + 1) <= L::I1D || lane + 64 * j < L::I1D) I1[lane + 64 * j] = i1v[j];
+  if (lane < 3 * Nfp) FM[lane] = fmv;
 #pragma unroll
   for (int j = 0; j < NGI; ++j) {
-    const int it = lane + 64 * j;
-    if (it < 16 * 3 * Nfp) {
-      const int e = it & 15, k = it >> 4, f = k / Nfp, i = k - f * Nfp;
-      const long gee = e0 + (e < cnt ? e : 0);
-      const int code = a.fcode[gee * 3 + f];
-      double v8[M];
-      if (code >= 0) {
-        const long nb = code >> 2;
-        const int nf = code & 3;
-        const double *src = a.q + (nb * Np + FM[nf * Nfp + (Nfp - 1 - i)]) * M;
+    const int k = 4 * j + lg;
+    if (4 * j + 4 <= 3 * Nfp || k < 3 * Nfp) {
 #pragma unroll
-        for (int v = 0; v < M; ++v) v8[v] = src[v];
-      } else {
-#pragma unroll
-        for (int v = 0; v < M; ++v) v8[v] = 0.0;
-      }
-#pragma unroll
-      for (int v = 0; v < M; ++v) PT[(k * M + v) * 16 + e] = XE(v8[v]);
+      for (int v = 0; v < M; ++v) PT[(k * M + v) * 16 + el] = XE(nbv[j][v]);
     }
   }
   wave_sync();
@@ -1235,7 +1264,11 @@ __global__ void __launch_bounds__((64 * RhsGroup<N, EQN, T>::W), (MinWaves<N, EQ
     }
   }
 
-#pragma unroll 2
+  // Two chunks per iteration, but one for 4-variable FP64 at N = 7, whose two
+  // chunks' operands no longer share 512 registers well (us per stage, one /
+  // two: N = 7, K = 80000 351 / 379; N = 6 247 / 244; N = 8 637 / 625).
+  constexpr int CHUNKS = IsF64<T>::value && N == 7 && M == 4 ? 1 : 2;
+#pragma unroll CHUNKS
   for (int cc = 0; cc < NCH; ++cc) {
     V4 qc[M];
 #pragma unroll
@@ -1454,24 +1487,6 @@ template <int N>
 struct LinOrder {
   static constexpr int NKP = (3 * Order<N>::Nfp + 3) / 4;   // k-steps of the face GEMM
 };
-
-// The neighbour's values at face node kf = f Nfp + i of element ge (its
-// node Fmask[nf][Nfp-1-i]); the element's own values there on boundary faces
-// (boundary_state sets them), of face 0 past the last face node.  Branch-free:
-// as branches, with the node numbers read from a table, each node's loads
-// waited for the table entry that its branch read, and with it for every load
-// before it.
-template <int N, int M>
-__device__ __forceinline__ void gather_face_node(const double *q, int kf, int code0, int code1,
-                                                 int code2, long ge, double *dst) {
-  constexpr int Np = Order<N>::Np, Nfp = N + 1;
-  const int f = kf < 3 * Nfp ? kf / Nfp : 0, i = kf < 3 * Nfp ? kf - f * Nfp : 0;
-  const int code = f == 0 ? code0 : (f == 1 ? code1 : code2);
-  const double *src = q + ((code >= 0 ? (long)(code >> 2) : ge) * Np +
-                           face_node<N>(code >= 0 ? code & 3 : 0, Nfp - 1 - i)) * M;
-#pragma unroll
-  for (int v = 0; v < M; ++v) dst[v] = src[v];
-}
 
 // Waves per SIMD requested from the register allocator (a lower bound: the
 // FP64 kernel fits three at N = 5 and four or more below N = 5).  FP64

@@ -1656,7 +1656,6 @@ static AdjArgs adj_args(apl_handle *h) {
   a.vert = h->d_vert;
   a.fcode = h->d_fcode;
   a.I1D = h->d_I1D;
-  a.fmask = h->d_fmask;
   a.Avc = h->d_adjops[0];
   a.Aart = h->d_adjops[1];
   a.Aast = h->d_adjops[2];
