@@ -78,7 +78,7 @@ VARIANTS = {
     "fp64": (0, 0), "fp32": (1, 0), "bf16x3": (2, 0),
     "fp64_cub": (0, 1), "fp32_cub": (1, 1), "bf16x3_cub": (2, 1),
     # the cubature form on a named kernel: MFMA at every order, or the
-    # vector-ALU kernel (N <= 3)
+    # vector-ALU kernels (N <= 3)
     "fp64_mfma": (0, 2), "fp32_mfma": (1, 2), "fp64_valu": (0, 3), "fp32_valu": (1, 3),
     # the nodal form of a linear flux on a named kernel
     "fp64_nmfma": (0, 4), "fp32_nmfma": (1, 4), "fp64_nvalu": (0, 5), "fp32_nvalu": (1, 5),
@@ -434,17 +434,23 @@ def calibrate_copy(mib, reps=10):
 
 def kernel_name(w, variant):
     """The engine's kernel for a variant: the nodal kernel for linear fluxes
-    (algorithm 0), the vector-ALU cubature kernel at N <= 3 in FP64/FP32
-    (algorithms 0, 1, 3; eight waves per group below 512 groups), else the
-    MFMA cubature kernel."""
+    (algorithm 0; in FP64 the even-odd one for the 8-variable system and small
+    TM meshes), the even-odd cubature kernel in FP64 at N <= 4, the vector-ALU
+    one in FP32 at N <= 3 (algorithms 0, 1, 3; eight waves per group below 512
+    groups), else the MFMA cubature kernel."""
     N = w.order
     prec, algo = VARIANTS[variant]
     ty = {"fp64": "double", "fp32": "float", "bf16x3": "apl::Bf16x3"}[variant.split("_")[0]]
     if w.linear and algo == 5:
         return "rhs_valu_linear_kernel<%d,%d,%d,%s>" % (N, w.eqn, w.flux, ty)
+    if w.linear and algo == 0 and prec == 0 and (
+            w.m == 8 or (w.K + 15) // 16 <= (512 if N <= 7 else 256)):
+        return "rhs_eo_linear_kernel<%d,%d,%d>" % (N, w.eqn, w.flux)
     if w.linear and algo in NODAL_ALGOS:
         return "rhs_linear_kernel<%d,%d,%d,%s>" % (N, w.eqn, w.flux, ty)
-    if N <= 3 and prec != 2 and algo != 2:
+    if N <= 4 and prec == 0 and algo != 2:
+        return "rhs_eo_kernel<%d,%d,%d>" % (N, w.eqn, w.flux)
+    if N <= 3 and prec == 1 and algo != 2:
         nw = 8 if (w.K + 63) // 64 < 512 else 4
         return "rhs_valu_kernel<%d,%d,%d,%s,%d>" % (N, w.eqn, w.flux, ty, nw)
     return "rhs_kernel<%d,%d,%d,%s>" % (N, w.eqn, w.flux, ty)
