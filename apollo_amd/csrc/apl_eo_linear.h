@@ -21,14 +21,14 @@
 //
 // Measured, us per LSERK4 stage, rhs_linear_kernel -> here:
 //   8 variables  K    1152         16200         45000          180000
-//     N = 2      11.7 ->  8.4   14.8 -> 13.2   28.9 -> 24.6    71 ->  68
-//     N = 4      16.9 -> 11.7   29.5 -> 24.5   59.1 -> 57.2   215 -> 188
-//     N = 6      27.3 -> 15.4   57.9 -> 43.6    134 -> 97     427 -> 334
-//     N = 8      44.7 -> 29.8    140 -> 100     296 -> 228    917 -> 706
+//     N = 2      11.7 ->  8.2   14.8 -> 12.5   28.9 -> 24.2      71 -> 64.7
+//     N = 4      16.9 -> 10.6   29.5 -> 24.1   59.1 -> 56.2     215 ->  173
+//     N = 6      27.3 -> 14.8   57.9 -> 43.8    134 -> 97.5     427 ->  319
+//     N = 8      44.7 -> 29.0    140 -> 98.5    296 ->  228     917 ->  708
 //   TM           K    1152          5000
 //     N = 3       9.1 ->  7.9   10.0 ->  8.8
-//     N = 5      13.5 -> 10.0   15.1 -> 11.1
-//     N = 7      19.2 -> 14.3   19.3 -> 14.8 (K = 3200)
+//     N = 5      13.5 ->  9.7   15.1 -> 11.3
+//     N = 7      19.2 -> 13.8   19.3 -> 14.2 (K = 3200)
 // Bound: K < 8192 the chain load -> fluxes -> products -> store; above it the
 // FP64 pipe from N = 5 on and the memory latency at two or three waves per
 // SIMD below.
