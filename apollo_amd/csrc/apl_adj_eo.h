@@ -30,7 +30,8 @@ namespace apl {
 // spill (5-variable Euler, N = 4: 315 us on MFMA, 558 here).
 constexpr bool adj_eo_order(int N, int M) { return N <= 4 && (N + 1) * (N + 2) / 2 * ((M + 1) / 2) <= 30; }
 
-// sqrt(x) as root() and 1 / (2 sqrt(x)) from the same iteration.
+// sqrt(x) as root() and 1 / (2 sqrt(x)) from the same iteration, for x >= 0
+// (0 gives about 2^-500 and 2^499; trace_vjp reports the rest).
 __device__ __forceinline__ double root_inv(double x, double &half_inv) {
   x = fmax(x, 0x1p-1000);
   const double y = __builtin_amdgcn_rsq(x);
@@ -106,9 +107,15 @@ __device__ __forceinline__ void euler_normal_vjp(double g1, const EulerPoint<EQN
 }
 
 // qMb = (dF*/dqM)^T nb and, with_p, qPb = (dF*/dqP)^T nb (num_flux_vjp; the
-// speed's derivative goes to the faster trace, qP on a tie).
+// speed's derivative goes to the faster trace, qP on a tie).  Returns whether
+// a wave speed that enters does not exist (gamma p / rho negative or NaN), or
+// has no derivative where that is used (gamma p / rho = 0): num_flux_vjp's
+// square roots and quotients are NaN or infinite there, root_inv's are not.
+// Compares alone, whose results are scalar masks: NaN and infinity carried
+// through the root keep more values live (N = 4, one wave: 84 bytes of scratch
+// against 56).
 template <int EQN, int FLUX>
-__device__ __forceinline__ void trace_vjp(const PhysParams &P, double nx, double ny, const double *qM,
+__device__ __forceinline__ bool trace_vjp(const PhysParams &P, double nx, double ny, const double *qM,
                                           const double *qP, const double *nb, bool with_p, double *qMb,
                                           double *qPb) {
   constexpr int M = Vars<EQN>::M;
@@ -117,9 +124,13 @@ __device__ __forceinline__ void trace_vjp(const PhysParams &P, double nx, double
     const double g = P.gamma, g1 = g - 1.0;
     const EulerPoint<EQN> sM(P, qM), sP(P, qP);
     double hs, ha, hsP, haP;
-    const double spM = root_inv(sM.k2, hs), aM = root_inv(g * sM.p * sM.ir, ha);
-    const double spP = root_inv(sP.k2, hsP), aP = root_inv(g * sP.p * sP.ir, haP);
+    const double xM = g * sM.p * sM.ir, xP = g * sP.p * sP.ir;
+    bool bad = !(xM >= 0.0) || !(xP >= 0.0);
+    const bool noneM = !(xM > 0.0), noneP = !(xP > 0.0);
+    const double spM = root_inv(sM.k2, hs), aM = root_inv(xM, ha);
+    const double spP = root_inv(sP.k2, hsP), aP = root_inv(xP, haP);
     const double cM = spM + aM, cP = spP + aP;
+    bad = bad || (cM > cP ? noneM : noneP && with_p);
     double b[M], jn = 0.0;
 #pragma unroll
     for (int c = 0; c < M; ++c) {
@@ -147,10 +158,12 @@ __device__ __forceinline__ void trace_vjp(const PhysParams &P, double nx, double
       for (int c = 0; c < M; ++c) qPb[c] -= l * b[c];
       speed(sP, spP, aP, hsP, haP, cM > cP ? 0.0 : jn, qPb);
     }
+    return bad;
   } else {
 #pragma unroll
     for (int c = 0; c < M; ++c) qMb[c] = qPb[c] = 0.0;
     num_flux_vjp<EQN, FLUX>(P, nx, ny, qM, qP, nb, qMb, qPb);
+    return false;
   }
 }
 
@@ -538,7 +551,7 @@ __global__ void __launch_bounds__(64 * W, (AdjEoWaves<N, EQN, W>::value))
         const double yg = vk[2 * va + 1] + sz * (vk[2 * vb2 + 1] - vk[2 * va + 1]);
         boundary_state<EQN, VTX>(*a.bc, -code - 1, a.t, xg, yg, nx, ny, qM, qP);
       }
-      trace_vjp<EQN, FLUX>(a.ph, nx, ny, qM, qP, nb, code < 0, qMb, qPb);
+      if (trace_vjp<EQN, FLUX>(a.ph, nx, ny, qM, qP, nb, code < 0, qMb, qPb)) ef |= EF_NAN;
       if (code < 0) boundary_vjp<EQN>(*a.bc, -code - 1, nx, ny, qPb, qMb);
       to_vars<M, MH>(qMb, xM, yM);
 #pragma unroll
