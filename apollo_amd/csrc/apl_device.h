@@ -210,8 +210,9 @@ __device__ __forceinline__ float recip(float x) {
 // ulp, in 9 instructions instead of the 17 of the IEEE-exact sequence (which
 // scales for subnormals and selects for 0 and infinity).  Arguments below
 // 2^-1000, 0 among them, return about 2^-500: next to nothing in a wave
-// speed.  A negative or NaN argument does the same (such a state raises its
-// own flag).
+// speed.  So do negative and NaN arguments, and infinity returns NaN: its
+// callers floor the state or flag it first (euler_prim, phys_flux), and a
+// state with an infinity or a NaN has a NaN flux.
 __device__ __forceinline__ double root(double x) {
   x = fmax(x, 0x1p-1000);
   const double y = __builtin_amdgcn_rsq(x);
@@ -401,7 +402,11 @@ __device__ __forceinline__ unsigned euler_lf_f32(const PhysParams &P, float nx, 
 // steps.  Roe is reproduced as Apollo computes it: the back-rotation assigns
 // the x-momentum slot twice, so it holds the y-momentum flux, and the
 // y-momentum slot keeps the 0 its buffer starts with.  Both zero the z
-// momentum flux.  *lam = max(|u| + c) of the two traces.
+// momentum flux.  The equation's floors act on both the primitive and the
+// conserved states that enter the speeds, the averages and the jumps
+// (wxeulereqn.cc:1324-1341): for HLL after the fluxes F and G took the traces
+// as they are, for Roe before.  (A floor of 0 raises a flag instead.)
+// *lam = max(|u| + c) of the two traces.
 template <int EQN, int FLUX>
 __device__ __forceinline__ unsigned euler_riemann_flux(const PhysParams &P, double nx, double ny,
                                                        const double *qMi, const double *qPi,
@@ -421,15 +426,37 @@ __device__ __forceinline__ unsigned euler_riemann_flux(const PhysParams &P, doub
   qP[1] = nx * qPi[1] + ny * qPi[2];
   qP[2] = -ny * qPi[1] + nx * qPi[2];
   double FM[M], GM[M], FP[M], GP[M];
-  unsigned ef = phys_flux<EQN, double>(P, qM, FM, GM);
-  ef |= phys_flux<EQN, double>(P, qP, FP, GP);
+  unsigned ef = 0;
+  if constexpr (FLUX == APL_FLUX_HLL) {
+    ef = phys_flux<EQN, double>(P, qM, FM, GM);
+    ef |= phys_flux<EQN, double>(P, qP, FP, GP);
+  }
+  if (P.min_dens != 0.0) {
+    if (qM[0] <= 0.0) qM[0] = P.min_dens;
+    if (qP[0] <= 0.0) qP[0] = P.min_dens;
+  }
   // rotated primitives: rho, u (normal), v, w, p
   const double iM = recip(qM[0]), iP = recip(qP[0]);
   const double uM = qM[1] * iM, vM = qM[2] * iM, wM = W ? qM[3] * iM : 0.0;
   const double uP = qP[1] * iP, vP = qP[2] * iP, wP = W ? qP[3] * iP : 0.0;
   const double mwM = W ? qM[3] : 0.0, mwP = W ? qP[3] : 0.0;
-  const double pM = (g - 1.) * (qM[IE] - 0.5 * (qM[1] * qM[1] + qM[2] * qM[2] + mwM * mwM) * iM);
-  const double pP = (g - 1.) * (qP[IE] - 0.5 * (qP[1] * qP[1] + qP[2] * qP[2] + mwP * mwP) * iP);
+  double pM = (g - 1.) * (qM[IE] - 0.5 * (qM[1] * qM[1] + qM[2] * qM[2] + mwM * mwM) * iM);
+  double pP = (g - 1.) * (qP[IE] - 0.5 * (qP[1] * qP[1] + qP[2] * qP[2] + mwP * mwP) * iP);
+  if (P.min_pres != 0.0) {
+    const double e0 = P.min_pres / (g - 1.);
+    if (pM <= 0.0) {
+      pM = P.min_pres;
+      qM[IE] = e0 + 0.5 * qM[0] * (uM * uM + vM * vM + wM * wM);
+    }
+    if (pP <= 0.0) {
+      pP = P.min_pres;
+      qP[IE] = e0 + 0.5 * qP[0] * (uP * uP + vP * vP + wP * wP);
+    }
+  }
+  if constexpr (FLUX == APL_FLUX_ROE) {
+    ef = phys_flux<EQN, double>(P, qM, FM, GM);
+    ef |= phys_flux<EQN, double>(P, qP, FP, GP);
+  }
   const double cM = root(g * pM * iM), cP = root(g * pP * iP);
   // Roe averages
   const double HM = (qM[IE] + pM) * iM, HP = (qP[IE] + pP) * iP;
@@ -508,7 +535,7 @@ __device__ __forceinline__ unsigned num_flux(const PhysParams &P, double nx, dou
     double fM[M], fP[M], cM, cP;
     unsigned ef = euler_normal_flux<EQN>(P, nx, ny, qM, fM, &cM);
     ef |= euler_normal_flux<EQN>(P, nx, ny, qP, fP, &cP);
-    const double l = fmax(cM, cP);   // root() gives no NaN
+    const double l = fmax(cM, cP);   // a NaN speed comes with a NaN flux
 #pragma unroll
     for (int c = 0; c < M; ++c) fs[c] = 0.5 * (fM[c] + fP[c] + l * (qM[c] - qP[c]));
     *lam = l;
