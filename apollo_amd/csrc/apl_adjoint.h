@@ -186,11 +186,20 @@ __device__ __forceinline__ void boundary_vjp(const BCTable &B, int idx, double n
                                              const double *qBCb, double *qMb) {
   constexpr int M = Vars<EQN>::M;
   const int kind = (idx >= 0 && idx < B.n) ? B.kind[idx] : APL_BC_COPY;
-  if (kind == APL_BC_ISENTROPIC_VORTEX) return;   // exterior state independent of q-
+  // exterior states independent of q-
+  if (kind == APL_BC_ISENTROPIC_VORTEX) return;
+  if ((EQN == APL_EQN_EULER5 || EQN == APL_EQN_EULER4) && kind == BC_FIXED) return;
   double t[M];
 #pragma unroll
   for (int c = 0; c < M; ++c) t[c] = qBCb[c];
-  if constexpr (EQN == APL_EQN_PHMAXWELL8) {
+  if constexpr (EQN == APL_EQN_EULER5 || EQN == APL_EQN_EULER4) {
+    if (kind == APL_BC_EULER_WALL) {   // the reflection is its own transpose; rho w = 0
+      const double bn = nx * qBCb[1] + ny * qBCb[2];
+      t[1] = qBCb[1] - 2. * bn * nx;
+      t[2] = qBCb[2] - 2. * bn * ny;
+      if constexpr (M == 5) t[3] = 0.0;
+    }
+  } else if constexpr (EQN == APL_EQN_PHMAXWELL8) {
     if (kind == APL_BC_MAXWELL_TM) {
       t[2] = -qBCb[2];
     } else if (kind == APL_BC_PEC) {

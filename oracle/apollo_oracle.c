@@ -1409,7 +1409,17 @@ static void bc_vjp(const orc_phys *ph, int bcnum, const double *nx, const double
   int idx = bcnum - 1;
   int kind = (idx >= 0 && idx < ph->nbc) ? ph->bc_kind[idx] : ORC_BC_NONE;
   switch (kind) {
-    case ORC_BC_VORTEX: break;
+    case ORC_BC_VORTEX:
+    case ORC_BC_EULER_INFLOW:
+    case ORC_BC_EULER_DIRICHLET: break;   /* qBC does not depend on qM */
+    case ORC_BC_EULER_WALL: {
+      double bn = nx[0] * qBCb[1] + nx[1] * qBCb[2];
+      qMb[0] += qBCb[0];
+      qMb[1] += qBCb[1] - 2. * bn * nx[0];
+      qMb[2] += qBCb[2] - 2. * bn * nx[1];
+      qMb[4] += qBCb[4];
+      break;
+    }
     case ORC_BC_TM:
       for (int c = 0; c < m; c++) qMb[c] += qBCb[c];
       qMb[2] -= 2.0 * qBCb[2];
