@@ -1313,9 +1313,11 @@ int apl_initial_dt(apl_handle *h, const double *q, double cfl, double *dt, int w
   if (p.eqn != APL_EQN_EULER5 && p.eqn != APL_EQN_EULER4) {
     maxSpeed = std::max(std::max(p.chi * p.c0, p.gamma_ph * p.c0), p.c0);
   } else if (where == APL_DEVICE) {
-    // q may come from the null stream, which a caller's own stream does not
-    // wait for
-    if (!h->own_stream) HIPCHK(h, hipStreamSynchronize(nullptr));
+    // A synchronous copy waits for every blocking stream, on any of which the
+    // caller may have filled q; the handle's stream alone waits for the null
+    // stream's work, or where it is the caller's for its own.
+    double first;
+    HIPCHK(h, hipMemcpy(&first, q, sizeof(double), hipMemcpyDeviceToHost));
     int n = 0;
     if (launch_roe_speed(h->stream, q, (long)nodes, M, p.gas_gamma, h->d_speed, &n))
       return fail(h, APL_ERR_HIP, "wave speed kernel launch failed");

@@ -264,7 +264,9 @@ int apl_rhs_noalloc(apl_handle *h, double t, const double *q, double *rhs, doubl
 int apl_limit(apl_handle *h, const double *q_in, double *q_out, int where);
 
 /* Initial-condition dt of WxNodalDG2dMethod::init (wxnodaldg2dmethod.cc:
- * 201-228): Roe wave speeds at every node, (2/3) cfl dtscale rmin / maxSpeed. */
+ * 201-228): Roe wave speeds at every node, (2/3) cfl dtscale rmin / maxSpeed.
+ * With APL_DEVICE it first waits for the work on every blocking stream, and
+ * runs on the handle's stream. */
 int apl_initial_dt(apl_handle *h, const double *q, double cfl, double *dt, int where);
 
 /* Low-storage RK4(5) (Carpenter & Kennedy 1994) over `nsteps` steps of a
