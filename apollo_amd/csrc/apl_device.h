@@ -590,7 +590,7 @@ __device__ __forceinline__ void store_euler5(const double *q5, double *q) {
 
 // A boundary state that depends on nothing but its parameters (inflow,
 // Dirichlet), as the kernels see it: BCTable.p holds the conserved state
-// (rho, rho u, rho v, rho w, E), formed once per call on the host.
+// (rho, rho u, rho v, rho w, E), formed on the host at creation.
 constexpr int BC_FIXED = 64;
 
 // Euler exterior states on the 5-variable state: isentropic vortex

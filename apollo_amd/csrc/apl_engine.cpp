@@ -205,12 +205,13 @@ static int dispatch_rhs(apl_handle *h, const RhsArgs &a) {
 }
 
 // The boundary list as the kernels read it: inflow (wxeulerinflowbc.cc:21-36)
-// and Dirichlet (wxeulerdirichletbc.cc:22-30) states formed here.
+// and Dirichlet (wxeulerdirichletbc.cc:22-30) states formed here.  A kind that
+// is none of the interface's is a copy, BC_FIXED's number too.
 static BCTable bc_table(const apl_params &p) {
   BCTable t;
   t.n = p.n_bc;
   for (int i = 0; i < APL_MAX_BC; ++i) {
-    t.kind[i] = p.bc[i].kind;
+    t.kind[i] = p.bc[i].kind == BC_FIXED ? (int)APL_BC_COPY : p.bc[i].kind;
     const double *s = p.bc[i].p;
     double *d = t.p[i];
     for (int j = 0; j < 8; ++j) d[j] = s[j];
