@@ -1794,8 +1794,9 @@ int launch_advance_time(hipStream_t s, double *t, double dt);
 // unsigned), which it clears for the next call.
 int launch_report(hipStream_t s, const double *in, int n, unsigned *err, double *pin);
 
-// pin[0] = sum of in[0 .. n) in a fixed order, to pinned host memory.
-int launch_sum_report(hipStream_t s, const double *in, int n, double *pin);
+// The values of in[0 .. n) that are not zero, in their order, to pinned host
+// memory: pin[0] = how many, pin[1 ..] the values.
+int launch_pack_report(hipStream_t s, const double *in, int n, double *pin);
 
 // part[b] = the largest squared Roe speed of the nodes of workgroup b
 // (SPEED_BLOCKS of them at most; returns how many in *nparts), Euler with m

@@ -81,7 +81,8 @@ struct apl_handle_s {
   LimTrace ltr{};
   bool ltr_is_state = false;   // trace slots = nodes 0..Np-1 of a 5-variable state
   // pinned host words the speed maximum and the flags are reported to (two
-  // doubles); flags_set: kernels ran since the flags were last cleared
+  // doubles), or an objective's partials (their number, then at most
+  // ceil(K/64)); flags_set: kernels ran since the flags were last cleared
   double *h_pin = nullptr;
   bool flags_set = true;
   // this device's copy of apl_rhs_noalloc's scratch array (not owned)
@@ -1013,7 +1014,8 @@ int apl_create(const apl_mesh *mesh, const apl_params *params, apl_handle **out)
   else if (params->precision == APL_PREC_FP32_MFMA) rc = upload_fragments<float>(h);
   else rc = upload_fragments_bf16x3(h);
   if (rc) return bail(rc);
-  if (hipHostMalloc((void **)&h->h_pin, 2 * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+  if (hipHostMalloc((void **)&h->h_pin, sizeof(double) * (2 + (size_t)h->K / 64), hipHostMallocDefault) !=
+      hipSuccess) {
     h->h_pin = nullptr;
     h->last_error = "pinned host allocation failed";
     return bail(APL_ERR_HIP);
@@ -1916,12 +1918,15 @@ int apl_objective_disc_sq(apl_handle *h, const double *q, int var, double xc, do
     default: rc = APL_ERR_ORDER;
   }
   if (rc) return fail(h, rc, "objective kernel launch failed");
-  if (launch_sum_report(h->stream, h->d_opart, nb, h->h_pin))
-    return fail(h, APL_ERR_HIP, "objective sum launch failed");
+  if (launch_pack_report(h->stream, h->d_opart, nb, h->h_pin))
+    return fail(h, APL_ERR_HIP, "objective report launch failed");
   if (dJdq && where == APL_HOST)
     HIPCHK(h, hipMemcpyAsync(dJdq, h->d_out, bytes, hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
-  *J = h->h_pin[0];
+  double sum = 0.0;
+  const int some = (int)h->h_pin[0];
+  for (int i = 1; i <= some; ++i) sum += h->h_pin[i];   // index order: deterministic
+  *J = sum;
   return APL_OK;
 }
 
