@@ -477,31 +477,32 @@ static bool make_eo_tables(const Operators &o, std::vector<double> &A1, std::vec
 
 // The folded operators of the nodal linear-flux form: D0 = Dt_r = A_r V_c,
 // D1 = Dt_s [Np x Np] and Lt = L blkdiag(I1D_f) [Np x 3Nfp] (see apl_device.h).
-static void fold_linear_operators(const Operators &o, std::vector<double> (&D)[2],
-                                  std::vector<double> &Lt) {
+// T: double or, for tables that are rounded once afterwards, long double.
+template <typename T>
+static void fold_linear_operators(const Operators &o, std::vector<T> (&D)[2], std::vector<T> &Lt) {
   const int Np = o.Np, Nc = o.Nc, Ng = o.Ng, Nfp = o.Nfp;
   D[0].assign((size_t)Np * Np, 0.0);
   D[1].assign((size_t)Np * Np, 0.0);
   Lt.assign((size_t)Np * 3 * Nfp, 0.0);
   for (int n = 0; n < Np; ++n) {
     // rows of A_r, A_s (V V^T Dr_c^T diag(w)) and L (V V^T I_f^T diag(gw))
-    std::vector<double> ar(Nc), as(Nc), lr(3 * Ng);
+    std::vector<T> ar(Nc), as(Nc), lr(3 * Ng);
     for (int c = 0; c < Nc; ++c) {
-      double sr = 0.0, ss = 0.0;
+      T sr = 0.0, ss = 0.0;
       for (int j = 0; j < Np; ++j) {
-        sr += o.VVT[(size_t)n * Np + j] * o.Drc[(size_t)c * Np + j];
-        ss += o.VVT[(size_t)n * Np + j] * o.Dsc[(size_t)c * Np + j];
+        sr += T(o.VVT[(size_t)n * Np + j]) * o.Drc[(size_t)c * Np + j];
+        ss += T(o.VVT[(size_t)n * Np + j]) * o.Dsc[(size_t)c * Np + j];
       }
       ar[c] = sr * o.cw[c];
       as[c] = ss * o.cw[c];
     }
     for (int k = 0; k < 3 * Ng; ++k) {
-      double sl = 0.0;
-      for (int j = 0; j < Np; ++j) sl += o.VVT[(size_t)n * Np + j] * o.If[(size_t)k * Np + j];
+      T sl = 0.0;
+      for (int j = 0; j < Np; ++j) sl += T(o.VVT[(size_t)n * Np + j]) * o.If[(size_t)k * Np + j];
       lr[k] = sl * o.gw[k % Ng];
     }
     for (int j = 0; j < Np; ++j) {
-      double sr = 0.0, ss = 0.0;
+      T sr = 0.0, ss = 0.0;
       for (int c = 0; c < Nc; ++c) {
         sr += ar[c] * o.Vc[(size_t)c * Np + j];
         ss += as[c] * o.Vc[(size_t)c * Np + j];
@@ -511,7 +512,7 @@ static void fold_linear_operators(const Operators &o, std::vector<double> (&D)[2
     }
     for (int f = 0; f < 3; ++f)
       for (int i = 0; i < Nfp; ++i) {
-        double sl = 0.0;
+        T sl = 0.0;
         for (int g = 0; g < Ng; ++g)
           sl += lr[f * Ng + g] * o.If[((size_t)f * Ng + g) * Np + o.fmask[f * Nfp + i]];
         Lt[(size_t)n * 3 * Nfp + f * Nfp + i] = sl;
@@ -566,11 +567,33 @@ static void make_linear_fragments(const Operators &o, std::vector<T> &A1, std::v
       }
 }
 
+// The mirror image of node n, and of face node k = f Nfp + i (Operators' order).
+static std::vector<int> eo_node_mirror(int N) {
+  std::vector<int> m((N + 1) * (N + 2) / 2);
+  for (int j = 0; j <= N; ++j)
+    for (int i = 0; i + j <= N; ++i) m[eo_node(N, i, j)] = eo_node(N, j, i);
+  return m;
+}
+
+static int eo_face_mirror(int N, int k) {
+  const int Nfp = N + 1, f = k / Nfp, i = k - f * Nfp;
+  return (f == 1 ? 1 : 2 - f) * Nfp + N - i;
+}
+
 // Operator tables of the even-odd nodal kernel (apl_eo_linear.h): A1 the volume
 // rows, A3 the lift rows, A2 the units' node lists (ints).  False as
 // make_eo_tables.
+//
+// The stored operators have the mirror symmetry only to the rounding of their
+// setup (2e-14 at N = 7), so the tables take the mean of each entry and its
+// mirror image, folded in long double.  What the symmetric part cannot hold is
+// felt where the terms cancel, a nearly constant state on a fine mesh: the rows
+// keep the stored operators' action on a constant flux exactly, its symmetric
+// part in the first axis node's entries, its antisymmetric part in that node's
+// second row, which no axis node needs otherwise.
 static bool make_eo_linear_tables(const Operators &o, std::vector<double> &A1,
                                   std::vector<int> &A2, std::vector<double> &A3) {
+  typedef long double ld;
   const int N = o.N, Np = o.Np, Nfp = o.Nfp;
   {
     std::vector<double> t1, t2, t3;
@@ -578,46 +601,71 @@ static bool make_eo_linear_tables(const Operators &o, std::vector<double> &A1,
   }
   std::vector<int> na, nb;
   const int NO = eo_node_list(N, na, nb), NE = (int)na.size();
-  std::vector<double> D[2], Lt;
+  std::vector<ld> D[2], Lt;
   fold_linear_operators(o, D, Lt);
-  auto rows = [&](std::vector<double> &t, const double *x, int stride, double se, double so) {
-    for (int i = 0; i < NE; ++i)
-      t.push_back(se * 0.5 * (x[(size_t)na[i] * stride] + x[(size_t)nb[i] * stride]));
-    for (int i = 0; i < NO; ++i)
-      t.push_back(so * 0.5 * (x[(size_t)na[i] * stride] - x[(size_t)nb[i] * stride]));
+  const std::vector<int> mir = eo_node_mirror(N);
+  auto Dm = [&](int a, int n) { return (D[0][(size_t)a * Np + n] + D[1][(size_t)mir[a] * Np + mir[n]]) / 2; };
+  auto Lm = [&](int a, int k) {
+    return (Lt[(size_t)a * 3 * Nfp + k] + Lt[(size_t)mir[a] * 3 * Nfp + eo_face_mirror(N, k)]) / 2;
+  };
+  // even and odd parts over the node list of a column x(a), scaled
+  auto rows = [&](std::vector<double> &t, ld s, auto x) {
+    for (int i = 0; i < NE; ++i) t.push_back(double(s * (x(na[i]) + x(nb[i])) / 2));
+    for (int i = 0; i < NO; ++i) t.push_back(double(s * (x(na[i]) - x(nb[i])) / 2));
   };
   const int ppu = EO_LPE / 2;
   A1.clear();
   A2.clear();
   A3.clear();
+  // what a constant Phi_r = 1 (Phi_s = 0) leaves in the rows, even and odd
+  // parts: Re, and Ro; a constant Phi_s leaves Re and -Ro
+  std::vector<ld> sum(Np, 0);
+  auto add = [&](const std::vector<double> &t, size_t at, ld even, ld odd) {
+    for (int i = 0; i < Np; ++i) sum[i] += (i < NE ? even : odd) * ld(t[at + i]);
+  };
   // volume pairs: node a, its mirror b (an axis node goes with itself, the
-  // second time with weight zero), padded to whole units
+  // second time with no weight but the first one's correction), padded to
+  // whole units
   for (int p = 0; p < (NE + ppu - 1) / ppu * ppu; ++p) {
     const int a = p < NE ? na[p] : 0, b = p < NE ? nb[p] : 0;
-    const double s1 = p < NE ? 1.0 : 0.0, s2 = p < NO ? 1.0 : 0.0;
-    rows(A1, &D[0][a], Np, s1, s1);
-    rows(A1, &D[0][b], Np, s2, s2);
+    rows(A1, p < NE ? 1 : 0, [&](int i) { return Dm(i, a); });
+    add(A1, A1.size() - Np, 1, 1);
+    rows(A1, p < NO ? 1 : 0, [&](int i) { return Dm(i, b); });
+    add(A1, A1.size() - Np, 1, 1);
     A2.push_back(a);
     A2.push_back(b);
   }
   // face-node pairs: bottom node i with left-side node N - i; hypotenuse node
-  // i with N - i (the middle one with itself, at half weight)
+  // i with N - i (the middle one with itself, at half weight).  Phi_r = 1 has
+  // S = 0, 1, -1 on the bottom, the hypotenuse, the left side
   const int NLP = Nfp + (Nfp + 1) / 2;
   for (int p = 0; p < (NLP + ppu - 1) / ppu * ppu; ++p) {
-    int k = 0, m = 0;
-    double s = 0.0;
-    if (p < Nfp) {
-      k = p;
-      m = 2 * Nfp + N - p;
-      s = 1.0;
-    } else if (p < NLP) {
-      k = Nfp + (p - Nfp);
-      m = Nfp + N - (p - Nfp);
-      s = k == m ? 0.5 : 1.0;
-    }
-    rows(A3, &Lt[k], 3 * Nfp, -s, -s);
+    const int k = p < NLP ? p : 0, m = p < NLP ? eo_face_mirror(N, k) : 0;
+    rows(A3, p < NLP ? (k == m ? -0.5L : -1) : 0, [&](int i) { return Lm(i, k); });
+    if (p < Nfp) add(A3, A3.size() - Np, -1, 1);
+    else add(A3, A3.size() - Np, 2, 0);
     A2.push_back(k);
     A2.push_back(m);
+  }
+  // the stored operators' action on Phi_r = 1 and on Phi_s = 1, less the rows'
+  auto stored = [&](int d, int a) {
+    ld s = 0;
+    for (int n = 0; n < Np; ++n) s += D[d][(size_t)a * Np + n];
+    for (int i = 0; i < Nfp; ++i)
+      s += Lt[(size_t)a * 3 * Nfp + (d == 0 ? 2 * Nfp : 0) + i] - Lt[(size_t)a * 3 * Nfp + Nfp + i];
+    return s;
+  };
+  double *first = &A1[(size_t)2 * NO * Np], *second = first + Np;   // the first axis node's rows
+  for (int i = 0; i < NE; ++i) {
+    const ld ra = stored(0, na[i]), rb = stored(0, nb[i]), sa = stored(1, na[i]), sb = stored(1, nb[i]);
+    const ld re = (ra + rb) / 2 - sum[i], se = (sa + sb) / 2 - sum[i];
+    first[i] = double(first[i] + (re + se) / 2);
+    second[i] = double((re - se) / 2);
+    if (i < NO) {
+      const ld ro = (ra - rb) / 2 - sum[NE + i], so = (sa - sb) / 2 + sum[NE + i];
+      first[NE + i] = double(first[NE + i] + (ro - so) / 2);
+      second[NE + i] = double((ro + so) / 2);
+    }
   }
   return true;
 }

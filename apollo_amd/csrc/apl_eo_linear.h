@@ -193,7 +193,7 @@ __global__ void __launch_bounds__(64 * W, (EoLinWaves<N, EQN>::value))
   constexpr int ES = C::ES, ESP = C::ESP, NVU = C::NVU, NFU = C::NFU, PPU = C::PPU, NT = 64 * W;
   constexpr EoNodes<N> ND{};
 
-  const cptr_t<double> TD = (cptr_t<double>)a.A1;     // [NVU PPU][VW]: De Do (a) | De Do (b)
+  const cptr_t<double> TD = (cptr_t<double>)a.A1;     // [NVU PPU][VW]: De Do (a) | De Do (b) or, on the axis, the correction
   const cptr_t<double> TL = (cptr_t<double>)a.A3;     // [NFU PPU][FW]: -Le -Lo
   const int *tab = (const int *)a.A2;                 // [TAB]
 
@@ -278,10 +278,13 @@ __global__ void __launch_bounds__(64 * W, (EoLinWaves<N, EQN>::value))
 #pragma unroll
     for (int s = 0; s < PPU; ++s) {
       const cptr_t<double> td = TD + (u * PPU + s) * C::VW;
+      // an axis node's second row acts on Phi_r - Phi_s and Phi_r + Phi_s, the
+      // parts that the mirror symmetry leaves out
+      const double sg = u * PPU + s < NO ? 1.0 : -1.0;
 #pragma unroll
       for (int j = 0; j < MH; ++j) {
         const double e1 = yr[2 * s][j] + ys[2 * s + 1][j], o1 = yr[2 * s][j] - ys[2 * s + 1][j];
-        const double e2 = yr[2 * s + 1][j] + ys[2 * s][j], o2 = yr[2 * s + 1][j] - ys[2 * s][j];
+        const double e2 = yr[2 * s + 1][j] + sg * ys[2 * s][j], o2 = yr[2 * s + 1][j] - sg * ys[2 * s][j];
 #pragma unroll
         for (int i = 0; i < NE; ++i) {
           Re[i][j] += td[i] * e1;
