@@ -200,7 +200,8 @@ __device__ __forceinline__ void eo_parts(const double *x, const int (&vo)[MH], d
 }
 
 // mu = V V^T x from the even and odd parts of x to LDS in the state's
-// layout (rows i = wave, wave + W, ...).  TV: [NE][NE] even, [NO][NO] odd.
+// layout (rows i = wave, wave + W, ...).  TV: [NE][NE] even, [NO][NO] odd, then
+// [NO] what the symmetry leaves out, of node MID's x.
 template <int N, int M, int MH, int W, int NE, int NO>
 __device__ __forceinline__ void eo_mass(const cptr_t<double> TV, const double (&e)[NE][MH],
                                         const double (&o)[NO][MH], const int (&vo)[MH], int wave,
@@ -211,7 +212,7 @@ __device__ __forceinline__ void eo_mass(const cptr_t<double> TV, const double (&
     if (W == 1 || i % W == wave) {
 #pragma unroll
       for (int j = 0; j < MH; ++j) {
-        double me = 0.0, mo = 0.0;
+        double me = 0.0, mo = i < NO ? TV[NE * NE + NO * NO + i] * e[EoNodes<N>::MID][j] : 0.0;
 #pragma unroll
         for (int k = 0; k < NE; ++k) me += TV[i * NE + k] * e[k][j];
         if (i < NO) {
@@ -271,6 +272,8 @@ __global__ void __launch_bounds__(64 * W, (AdjEoWaves<N, EQN, W>::value))
 
   const cptr_t<double> TP = (cptr_t<double>)a.TP;     // rows of apl_eo.h
   const cptr_t<double> TX = TP + NPR * C::VW;
+  const cptr_t<double> TD = TX + C::NAX * C::XW;      // [NV][2] what the symmetry leaves out of a
+                                                      // unit's points, of node MID's weight
   const cptr_t<double> TI = (cptr_t<double>)a.TI;     // [NFU][Nfp] Ie Io, abscissae, weights [NFU]
 
   const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
@@ -370,7 +373,8 @@ __global__ void __launch_bounds__(64 * W, (AdjEoWaves<N, EQN, W>::value))
       double x[MH], y[MH], q[M], rx[MH], ry[MH], sx[MH], sy[MH];
 #pragma unroll
       for (int j = 0; j < MH; ++j) {
-        double ev = 0.0, od = 0.0, e1 = 0.0, o1 = 0.0, e2 = 0.0, o2 = 0.0;
+        double ev = 0.0, od = 0.0, e1 = 0.0, e2 = 0.0;
+        double o1 = TD[2 * c] * Le[EoNodes<N>::MID][j], o2 = TD[2 * c + 1] * Le[EoNodes<N>::MID][j];
 #pragma unroll
         for (int i = 0; i < NE; ++i) {
           ev += tv[i] * Qe[i][j];
@@ -416,7 +420,8 @@ __global__ void __launch_bounds__(64 * W, (AdjEoWaves<N, EQN, W>::value))
       double x[MH], y[MH], q[M], rx[MH], ry[MH], sx[MH], sy[MH];
 #pragma unroll
       for (int j = 0; j < MH; ++j) {
-        double e1 = 0.0, o1 = 0.0, e2 = 0.0, o2 = 0.0;
+        double e1 = 0.0, e2 = 0.0;
+        double o1 = TD[2 * c] * Le[EoNodes<N>::MID][j], o2 = TD[2 * c + 1] * Le[EoNodes<N>::MID][j];
         x[j] = y[j] = 0.0;
 #pragma unroll
         for (int i = 0; i < NE; ++i) {

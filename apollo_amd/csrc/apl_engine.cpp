@@ -306,26 +306,27 @@ static int report(apl_handle *h, const double *part = nullptr, int n = 0, double
 }
 
 // The folded operators of the cubature form: A_r = V V^T Dr_c^T diag(w)
-// and A_s likewise [Np x Nc], L = V V^T I_f^T diag(gw) [Np x 3Ng].
-static void fold_operators(const Operators &o, std::vector<double> &Ar, std::vector<double> &As,
-                           std::vector<double> &L) {
+// and A_s likewise [Np x Nc], L = V V^T I_f^T diag(gw) [Np x 3Ng].  T: double
+// or, for tables that are rounded once afterwards, long double.
+template <typename T>
+static void fold_operators(const Operators &o, std::vector<T> &Ar, std::vector<T> &As, std::vector<T> &L) {
   const int Np = o.Np, Nc = o.Nc, Ng = o.Ng;
   Ar.assign((size_t)Np * Nc, 0.0);
   As.assign((size_t)Np * Nc, 0.0);
   L.assign((size_t)Np * 3 * Ng, 0.0);
   for (int n = 0; n < Np; ++n) {
     for (int c = 0; c < Nc; ++c) {
-      double sr = 0.0, ss = 0.0;
+      T sr = 0.0, ss = 0.0;
       for (int j = 0; j < Np; ++j) {
-        sr += o.VVT[(size_t)n * Np + j] * o.Drc[(size_t)c * Np + j];
-        ss += o.VVT[(size_t)n * Np + j] * o.Dsc[(size_t)c * Np + j];
+        sr += T(o.VVT[(size_t)n * Np + j]) * o.Drc[(size_t)c * Np + j];
+        ss += T(o.VVT[(size_t)n * Np + j]) * o.Dsc[(size_t)c * Np + j];
       }
       Ar[(size_t)n * Nc + c] = sr * o.cw[c];
       As[(size_t)n * Nc + c] = ss * o.cw[c];
     }
     for (int k = 0; k < 3 * Ng; ++k) {
-      double s = 0.0;
-      for (int j = 0; j < Np; ++j) s += o.VVT[(size_t)n * Np + j] * o.If[(size_t)k * Np + j];
+      T s = 0.0;
+      for (int j = 0; j < Np; ++j) s += T(o.VVT[(size_t)n * Np + j]) * o.If[(size_t)k * Np + j];
       L[(size_t)n * 3 * Ng + k] = s * o.gw[k % Ng];
     }
   }
@@ -402,13 +403,42 @@ static int eo_node_list(int N, std::vector<int> &na, std::vector<int> &nb) {
   return NO;
 }
 
+// The mirror image of node n, and of face node k = f Nfp + i (Operators' order).
+static std::vector<int> eo_node_mirror(int N) {
+  std::vector<int> m((N + 1) * (N + 2) / 2);
+  for (int j = 0; j <= N; ++j)
+    for (int i = 0; i + j <= N; ++i) m[eo_node(N, i, j)] = eo_node(N, j, i);
+  return m;
+}
+
+static int eo_face_mirror(int N, int k) {
+  const int Nfp = N + 1, f = k / Nfp, i = k - f * Nfp;
+  return (f == 1 ? 1 : 2 - f) * Nfp + N - i;
+}
+
 // Operator tables of the even-odd kernel (apl_eo.h).  False if the order's
 // nodes, faces or cubature rule do not have the mirror symmetry the kernel
 // is built on.
+//
+// The stored operators have it only to the rounding of their setup (2e-15 of
+// the largest entry at N = 4), so the tables take the mean of each entry and
+// its mirror image, folded in long double.  What the symmetric part cannot hold
+// is felt where the terms cancel, a nearly constant state on a fine mesh: the
+// rows keep the stored operators' action on a constant state exactly (fluxes of
+// degree 1 in the state), its symmetric part in the first axis point's entries,
+// its antisymmetric part in one more row that acts on Phi_r - Phi_s (even) and
+// Phi_r + Phi_s (odd) of that point.
+//
+// With `mass` (M 1, the mass matrix's row sums) the tables are the adjoint's,
+// whose terms cancel for weights lam / J = M 1: instead, each point keeps its
+// column's action on those exactly, its symmetric part in the entry of the axis
+// node next to the centroid (EoNodes::MID), its antisymmetric part in one more
+// number per point, [NV][2] after the rows, that multiplies this node's weight.
 static bool make_eo_tables(const Operators &o, std::vector<double> &A1, std::vector<double> &A2,
-                           std::vector<double> &A3) {
+                           std::vector<double> &A3, const std::vector<double> *mass = nullptr) {
+  typedef long double ld;
   const int N = o.N, Np = o.Np, Nc = o.Nc, Ng = o.Ng, Nfp = o.Nfp;
-  const double tol = 1e-11;
+  const double tol = 1e-14;
   for (int f = 0; f < 3; ++f)
     for (int i = 0; i < Nfp; ++i)
       if (o.fmask[f * Nfp + i] != eo_fmask(N, f, i)) return false;
@@ -416,62 +446,142 @@ static bool make_eo_tables(const Operators &o, std::vector<double> &A1, std::vec
   const int NO = eo_node_list(N, na, nb), NE = (int)na.size();
   for (int i = 0; i < NE; ++i)
     if (std::fabs(o.r[na[i]] - o.s[nb[i]]) + std::fabs(o.s[na[i]] - o.r[nb[i]]) > tol) return false;
-  std::vector<int> pc, pm, ax;   // point pairs and axis points
+  std::vector<int> mir = eo_node_mirror(N), cm(Nc);   // mirror images of nodes, points
+  std::vector<int> pc, ax;                            // first points of the pairs, axis points
   for (int c = 0; c < Nc; ++c) {
     int m = -1;
     for (int k = 0; k < Nc; ++k)
       if (std::fabs(o.cr[c] - o.cs[k]) + std::fabs(o.cs[c] - o.cr[k]) < tol) m = k;
     if (m < 0 || std::fabs(o.cw[c] - o.cw[m]) > tol) return false;
+    cm[c] = m;
     if (m == c) ax.push_back(c);
-    if (m > c) {
-      pc.push_back(c);
-      pm.push_back(m);
-    }
+    if (m > c) pc.push_back(c);
   }
   if ((int)ax.size() != eo_axis_points(N) || (int)(2 * pc.size() + ax.size()) != Nc) return false;
-  std::vector<double> Ar, As, L;
+  std::vector<ld> Ar, As, L;
   fold_operators(o, Ar, As, L);
+  auto Vm = [&](int c, int n) { return ((ld)o.Vc[(size_t)c * Np + n] + o.Vc[(size_t)cm[c] * Np + mir[n]]) / 2; };
+  auto Am = [&](int n, int c) { return (Ar[(size_t)n * Nc + c] + As[(size_t)mir[n] * Nc + cm[c]]) / 2; };
   // even and odd parts over the node list of a point's row (V) or column (A, L)
-  auto halves = [&](std::vector<double> &t, const double *x, int stride, double scale, bool even, bool odd) {
-    if (even)
-      for (int i = 0; i < NE; ++i)
-        t.push_back(scale * (i < NO ? 0.5 * (x[(size_t)na[i] * stride] + x[(size_t)nb[i] * stride])
-                                    : x[(size_t)na[i] * stride]));
+  auto halves = [&](std::vector<double> &t, ld scale, bool odd, auto x) {
+    for (int i = 0; i < NE; ++i) t.push_back(double(scale * (x(na[i]) + x(nb[i])) / 2));
     if (odd)
-      for (int i = 0; i < NO; ++i)
-        t.push_back(scale * 0.5 * (x[(size_t)na[i] * stride] - x[(size_t)nb[i] * stride]));
+      for (int i = 0; i < NO; ++i) t.push_back(double(scale * (x(na[i]) - x(nb[i])) / 2));
   };
+  // what Phi_r = 1 and Phi_s = 1 of a constant state leave in the rows, in
+  // even and odd parts
+  std::vector<ld> sr(Np, 0), ss(Np, 0);
+  auto add = [&](std::vector<ld> &sum, const std::vector<double> &t, size_t at, ld even, ld odd) {
+    for (int i = 0; i < Np; ++i) sum[i] += (i < NE ? even : odd) * (ld)t[at + i];
+  };
+  // the interpolation of 1 by an even part
+  auto one = [](const std::vector<double> &t, size_t at, int pairs, int all) {
+    ld s = 0;
+    for (int i = 0; i < all; ++i) s += (i < pairs ? 2 : 1) * (ld)t[at + i];
+    return s;
+  };
+  std::vector<double> more;
   A1.clear();
-  for (size_t p = 0; p < pc.size(); ++p) {
-    halves(A1, &o.Vc[(size_t)pc[p] * Np], 1, 1.0, true, true);
-    halves(A1, &Ar[pc[p]], Nc, 1.0, true, true);
-    halves(A1, &Ar[pm[p]], Nc, 1.0, true, true);
+  auto point = [&](int c, ld weight, ld rho) {
+    halves(A1, weight, true, [&](int n) { return Am(n, c); });
+    add(sr, A1, A1.size() - Np, rho, rho);
+    add(ss, A1, A1.size() - Np, rho, -rho);
+    if (!mass) return;
+    const std::vector<double> &m = *mass;
+    double *col = &A1[A1.size() - Np];
+    ld even = 0, odd = 0, tr = 0, ts = 0;
+    for (int i = 0; i < NE; ++i) even += col[i] * (i < NO ? (ld)m[na[i]] + m[nb[i]] : (ld)m[na[i]]);
+    for (int i = 0; i < NO; ++i) odd += col[NE + i] * ((ld)m[na[i]] - m[nb[i]]);
+    for (int n = 0; n < Np; ++n) {
+      tr += weight * Ar[(size_t)n * Nc + c] * m[n];
+      ts += weight * As[(size_t)n * Nc + cm[c]] * m[n];
+    }
+    const int mid = NO + (N + 1) / 3;
+    col[mid] = double(col[mid] + ((tr + ts) / 2 - even) / m[na[mid]]);
+    more.push_back(double(((tr - ts) / 2 - odd) / m[na[mid]]));
+  };
+  for (int c : pc) {
+    halves(A1, 1, true, [&](int n) { return Vm(c, n); });
+    const ld rho = one(A1, A1.size() - Np, NO, NE);
+    point(c, 1, rho);
+    point(cm[c], 1, rho);
   }
+  const size_t axis = A1.size();
   for (size_t p = 0; p < ax.size(); p += 2) {
     const bool two = p + 1 < ax.size();   // a point left over goes with itself, weight zero
     const int c1 = ax[p], c2 = two ? ax[p + 1] : c1;
-    halves(A1, &o.Vc[(size_t)c1 * Np], 1, 1.0, true, false);
-    halves(A1, &o.Vc[(size_t)c2 * Np], 1, 1.0, true, false);
-    halves(A1, &Ar[c1], Nc, 1.0, true, true);
-    halves(A1, &Ar[c2], Nc, two ? 1.0 : 0.0, true, true);
+    halves(A1, 1, false, [&](int n) { return Vm(c1, n); });
+    halves(A1, 1, false, [&](int n) { return Vm(c2, n); });
+    const ld r1 = one(A1, A1.size() - 2 * NE, NO, NE), r2 = one(A1, A1.size() - NE, NO, NE);
+    point(c1, 1, r1);
+    point(c2, two ? 1 : 0, r2);
   }
+  // the face interpolation is the same on the three faces (their mean); its
+  // even and odd parts per Gauss pair, then the abscissae
+  A2.clear();
+  for (int g = 0; g < Ng / 2; ++g) {
+    auto at = [&](int i) {
+      ld x = 0;
+      for (int f = 0; f < 3; ++f)
+        x += (ld)o.If[((size_t)f * Ng + g) * Np + o.fmask[f * Nfp + i]] +
+             o.If[((size_t)f * Ng + Ng - 1 - g) * Np + o.fmask[f * Nfp + Nfp - 1 - i]];
+      return x / 6;
+    };
+    for (int i = 0; i < (Nfp + 1) / 2; ++i)
+      A2.push_back(double(2 * i + 1 == Nfp ? at(i) : (at(i) + at(Nfp - 1 - i)) / 2));
+    for (int i = 0; i < Nfp / 2; ++i) A2.push_back(double((at(i) - at(Nfp - 1 - i)) / 2));
+  }
+  // S of Phi_r = 1 is 0, 1, -1 times the interpolated 1 on the bottom, the
+  // hypotenuse, the left side; of Phi_s = 1 it is -1, 1, 0
   A3.clear();
   for (int f = 0; f < 3; ++f)
     for (int g = 0; g < Ng / 2; ++g) {
-      halves(A3, &L[f * Ng + g], 3 * Ng, -1.0, true, true);
-      halves(A3, &L[f * Ng + Ng - 1 - g], 3 * Ng, -1.0, true, true);
+      const ld x = one(A2, (size_t)g * Nfp, Nfp / 2, (Nfp + 1) / 2);
+      for (int k : {g, Ng - 1 - g}) {
+        halves(A3, -1, true, [&](int n) { return L[(size_t)n * 3 * Ng + f * Ng + k]; });
+        const ld tr = f == 0 ? 0 : f == 1 ? x : -x, ts = f == 0 ? -x : f == 1 ? x : 0;
+        add(sr, A3, A3.size() - Np, tr, tr);
+        add(ss, A3, A3.size() - Np, ts, ts);
+      }
     }
-  // the face interpolation is the same on the three faces; its even and odd
-  // parts per Gauss pair, then the abscissae
-  A2.clear();
-  for (int g = 0; g < Ng / 2; ++g) {
-    const double *x = &o.If[(size_t)g * Np];
-    auto at = [&](int i) { return x[o.fmask[i]]; };
-    for (int i = 0; i < (Nfp + 1) / 2; ++i)
-      A2.push_back(2 * i + 1 == Nfp ? at(i) : 0.5 * (at(i) + at(Nfp - 1 - i)));
-    for (int i = 0; i < Nfp / 2; ++i) A2.push_back(0.5 * (at(i) - at(Nfp - 1 - i)));
-  }
   for (int g = 0; g < Ng / 2; ++g) A2.push_back(o.gz[g]);
+  if (mass) {
+    A1.insert(A1.end(), more.begin(), more.end());
+    return true;
+  }
+  // the stored operators' action on Phi_r = 1 and on Phi_s = 1, less the rows';
+  // half of a face flux is the neighbour's, from any of its three faces' rows
+  auto row = [&](const std::vector<double> &A, int k) {
+    ld x = 0;
+    for (int j = 0; j < Np; ++j) x += A[(size_t)k * Np + j];
+    return x;
+  };
+  auto face = [&](int f, int g) {
+    ld other = 0;
+    for (int f2 = 0; f2 < 3; ++f2) other += row(o.If, f2 * Ng + Ng - 1 - g);
+    return (row(o.If, f * Ng + g) + other / 3) / 2;
+  };
+  auto stored = [&](int d, int n) {
+    const int out = d == 0 ? 2 : 0;
+    ld x = 0;
+    for (int c = 0; c < Nc; ++c) x += (d == 0 ? Ar : As)[(size_t)n * Nc + c] * row(o.Vc, c);
+    for (int g = 0; g < Ng; ++g)
+      x += L[(size_t)n * 3 * Ng + out * Ng + g] * face(out, g) - L[(size_t)n * 3 * Ng + Ng + g] * face(1, g);
+    return x;
+  };
+  A1.resize(A1.size() + Np, 0.0);
+  double *first = &A1[axis + 2 * NE], *last = &A1[A1.size() - Np];
+  for (int i = 0; i < NE; ++i) {
+    const ld ra = stored(0, na[i]), rb = stored(0, nb[i]), sa = stored(1, na[i]), sb = stored(1, nb[i]);
+    const ld re = (ra + rb) / 2 - sr[i], se = (sa + sb) / 2 - ss[i];
+    first[i] = double(first[i] + (re + se) / 2);
+    last[i] = double((re - se) / 2);
+    if (i < NO) {
+      const ld ro = (ra - rb) / 2 - sr[NE + i], so = (sa - sb) / 2 - ss[NE + i];
+      first[NE + i] = double(first[NE + i] + (ro - so) / 2);
+      last[NE + i] = double((ro + so) / 2);
+    }
+  }
   return true;
 }
 
@@ -565,19 +675,6 @@ static void make_linear_fragments(const Operators &o, std::vector<T> &A1, std::v
         const int n = 16 * rt + (l & 15), k = 4 * ks + (l >> 4);
         if (n < Np && k < 3 * Nfp) A3[((size_t)rt * NKP + ks) * 64 + l] = T(-Lt[(size_t)n * 3 * Nfp + k]);
       }
-}
-
-// The mirror image of node n, and of face node k = f Nfp + i (Operators' order).
-static std::vector<int> eo_node_mirror(int N) {
-  std::vector<int> m((N + 1) * (N + 2) / 2);
-  for (int j = 0; j <= N; ++j)
-    for (int i = 0; i + j <= N; ++i) m[eo_node(N, i, j)] = eo_node(N, j, i);
-  return m;
-}
-
-static int eo_face_mirror(int N, int k) {
-  const int Nfp = N + 1, f = k / Nfp, i = k - f * Nfp;
-  return (f == 1 ? 1 : 2 - f) * Nfp + N - i;
 }
 
 // Operator tables of the even-odd nodal kernel (apl_eo_linear.h): A1 the volume
@@ -1650,21 +1747,51 @@ static int upload_adjoint_fragments(apl_handle *h) {
 
 // Tables of the even-odd adjoint kernels (apl_adj_eo.h): the point rows of
 // apl_eo.h, its face interpolation with the Gauss weights, and V V^T on even
-// and odd parts.
+// and odd parts, which keeps its action on M 1 as the points do: the
+// antisymmetric part in [NO] numbers after its rows.
 static int upload_adjoint_eo(apl_handle *h) {
+  typedef long double ld;
   const Operators &o = h->ops;
-  std::vector<double> A1, A2, A3, TV;
-  if (!make_eo_tables(o, A1, A2, A3)) return fail(h, APL_ERR_ORDER, "the order's tables lack the mirror symmetry");
+  const int Np = o.Np;
+  std::vector<double> A1, A2, A3, TV, M((size_t)Np * Np), m(Np, 0.0);
+  if (!invert(Np, o.VVT.data(), M.data())) return fail(h, APL_ERR_ORDER, "mass matrix inversion failed");
+  for (int i = 0; i < Np; ++i)
+    for (int j = 0; j < Np; ++j) m[i] += M[(size_t)i * Np + j];
+  if (!make_eo_tables(o, A1, A2, A3, &m))
+    return fail(h, APL_ERR_ORDER, "the order's tables lack the mirror symmetry");
   for (int g = 0; g < o.Ng / 2; ++g) A2.push_back(o.gw[g]);
   std::vector<int> na, nb;
   const int NO = eo_node_list(o.N, na, nb), NE = (int)na.size();
-  const double *V = o.VVT.data();
-  for (int i = 0; i < NE; ++i)
-    for (int j = 0; j < NE; ++j)
-      TV.push_back(0.5 * (V[(size_t)na[i] * o.Np + na[j]] + V[(size_t)na[i] * o.Np + nb[j]]));
-  for (int i = 0; i < NO; ++i)
-    for (int j = 0; j < NO; ++j)
-      TV.push_back(0.5 * (V[(size_t)na[i] * o.Np + na[j]] - V[(size_t)na[i] * o.Np + nb[j]]));
+  auto V = [&](int i, int j) { return (ld)o.VVT[(size_t)i * Np + j]; };
+  // the mean of an entry and its mirror image, as make_eo_tables
+  auto entry = [&](int i, int j, int sign) {
+    return double((V(na[i], na[j]) + V(nb[i], nb[j]) + sign * (V(na[i], nb[j]) + V(nb[i], na[j]))) / 4);
+  };
+  auto stored = [&](int i) {
+    ld x = 0;
+    for (int n = 0; n < Np; ++n) x += V(i, n) * m[n];
+    return x;
+  };
+  const int mid = NO + (o.N + 1) / 3;
+  for (int i = 0; i < NE; ++i) {
+    ld even = 0;
+    for (int j = 0; j < NE; ++j) {
+      TV.push_back(entry(i, j, 1));
+      even += TV.back() * (j < NO ? (ld)m[na[j]] + m[nb[j]] : (ld)m[na[j]]);
+    }
+    double &at = TV[TV.size() - NE + mid];
+    at = double(at + ((stored(na[i]) + stored(nb[i])) / 2 - even) / m[na[mid]]);
+  }
+  std::vector<double> more;
+  for (int i = 0; i < NO; ++i) {
+    ld odd = 0;
+    for (int j = 0; j < NO; ++j) {
+      TV.push_back(entry(i, j, -1));
+      odd += TV.back() * ((ld)m[na[j]] - m[nb[j]]);
+    }
+    more.push_back(double(((stored(na[i]) - stored(nb[i])) / 2 - odd) / m[na[mid]]));
+  }
+  TV.insert(TV.end(), more.begin(), more.end());
   const std::vector<double> *src[3] = {&A1, &A2, &TV};
   int rc;
   for (int i = 0; i < 3; ++i)

@@ -52,6 +52,7 @@ struct EoNodes {
   static constexpr int NX = N / 2 + 1;          // nodes on the axis
   static constexpr int NO = (Np - NX) / 2;      // pairs
   static constexpr int NE = NO + NX;
+  static constexpr int MID = NO + (N + 1) / 3;  // the axis node nearest to the centroid
   int a[NE] = {}, b[NE] = {};
   constexpr EoNodes() {
     int k = 0;
@@ -273,7 +274,8 @@ __global__ void __launch_bounds__(64 * W, (EoWaves<N, EQN, W>::value))
 
   // operator tables, read with wave-uniform indices (scalar loads)
   const cptr_t<double> TP = (cptr_t<double>)a.A1;     // [NPR][VW]: Ve Vo | Ae Ao (c) | Ae Ao (c')
-  const cptr_t<double> TX = TP + NPR * C::VW;         // [NAX][XW]: Ve(c1) Ve(c2) | Ae Ao (c1) | Ae Ao (c2)
+  const cptr_t<double> TX = TP + NPR * C::VW;         // [NAX][XW]: Ve(c1) Ve(c2) | Ae Ao (c1) | Ae Ao (c2), then
+                                                      // [Np]: the first axis point's correction
   const cptr_t<double> TF = (cptr_t<double>)a.A3;     // [3 NFU][FW]: -Le -Lo (g) | -Le -Lo (Ng-1-g)
   const cptr_t<double> TI = (cptr_t<double>)a.A2;     // [NFU][Nfp]: Ie Io (g), then the abscissae [NFU]
 
@@ -452,6 +454,16 @@ __global__ void __launch_bounds__(64 * W, (EoWaves<N, EQN, W>::value))
         for (int i = 0; i < NO; ++i) {
           Ro[i][j] += ta[NE + i] * o1[j];
           Ro[i][j] += ta[Np + NE + i] * o2[j];
+        }
+      }
+      if (c == NPR) {   // the parts that the mirror symmetry leaves out
+        const cptr_t<double> tc = TX + C::NAX * C::XW;
+#pragma unroll
+        for (int j = 0; j < MH; ++j) {
+#pragma unroll
+          for (int i = 0; i < NE; ++i) Re[i][j] += tc[i] * o1[j];
+#pragma unroll
+          for (int i = 0; i < NO; ++i) Ro[i][j] += tc[NE + i] * e1[j];
         }
       }
     }

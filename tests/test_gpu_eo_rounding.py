@@ -113,3 +113,58 @@ def test_eo_nodal_rounding(N, eqn):
     here, mfma = _errors(N, eqn, (E.ALGO_AUTO, E.ALGO_NODAL_MFMA))
     print("N %d: even-odd %.2e, MFMA %.2e, ratio %.2f" % (N, here, mfma, here / mfma))
     assert here <= np.sqrt(2.0) * mfma
+
+
+@pytest.mark.parametrize("N", range(1, 5))
+@pytest.mark.parametrize("eqn", [E.EQN_EULER4, E.EQN_EULER5])
+def test_eo_cubature_rounding(N, eqn):
+    here, mfma = _errors(N, eqn, (E.ALGO_CUBATURE, E.ALGO_CUBATURE_MFMA))
+    print("N %d: even-odd %.2e, MFMA %.2e, ratio %.2f" % (N, here, mfma, here / mfma))
+    assert here <= np.sqrt(2.0) * mfma
+
+
+def _adjoint(N, mesh, geom, lam):
+    """J^T lam of the TM system with the LF flux, in long double from the stored operators and geometry."""
+    op = lambda k: E.host_operator(N, k).astype(LD)  # noqa: E731
+    w, gw, Np = op(5), op(7), op(8).size
+    Nc, Ng = w.size, gw.size
+    V, Dr, Ds = (op(k).reshape(Nc, Np) for k in (0, 1, 2))
+    If, VVT = op(3).reshape(3 * Ng, Np), op(4).reshape(Np, Np)
+    F, G, _ = _flux(E.EQN_MAXWELL_TM3, np.eye(3).astype(LD))     # rows: the fluxes of the unit states
+    t = lambda A, x: np.einsum("ij,kim->kjm", A, x)  # noqa: E731
+    jrx, jsx, jry, jsy = ((geom[:, 4] * geom[:, k]).astype(LD)[:, None, None] for k in range(4))
+    lh = lam.astype(LD) / geom[:, 4].astype(LD)[:, None, None]
+    pr, ps = t((VVT @ Dr.T) * w, lh), t((VVT @ Ds.T) * w, lh)
+    out = t(V, (jrx * pr + jsx * ps) @ F.T + (jry * pr + jsy * ps) @ G.T)
+    n = geom[:, 5:].reshape(mesh.K, 3, 1, 3).astype(LD)
+    S = -n[..., 2:] * t((VVT @ If.T) * np.tile(gw, 3), lh).reshape(mesh.K, 3, Ng, 3)
+    et = E.host_connectivity(mesh).reshape(mesh.K, 3, 2)
+    half = (S - S[et[:, :, 0], et[:, :, 1]][:, :, ::-1]) / 2
+    f = n[..., :1] * (half @ F.T) + n[..., 1:2] * (half @ G.T) + half
+    return out + t(If, f.reshape(mesh.K, 3 * Ng, 3))
+
+
+def test_eo_adjoint_rounding():
+    """The adjoint of weights M mu with smooth mu, whose terms cancel as the
+    forward RHS's do, more so with the order: the even-odd kernels (N <= 4) are
+    no farther from the long double value than the MFMA kernel at N = 5."""
+    err = {}
+    for N in range(1, 6):
+        mesh, params = _case(N, E.EQN_MAXWELL_TM3, E.FLUX_LF)
+        case = Case(mesh, params(E.ALGO_AUTO))
+        eng = E.Engine(mesh, case.params)
+        geom = eng.geometry()[0].reshape(mesh.K, 14)
+        mass = np.linalg.inv(E.host_operator(N, 4).reshape(case.ops.Np, case.ops.Np))
+        total = 0.0
+        for seed in range(3):
+            q = _state(case, 3, False, seed)
+            lam = np.ascontiguousarray(geom[:, 4, None, None] * np.einsum("ij,kjm->kim", mass, q))
+            out = np.zeros_like(q)
+            eng.adjoint_rhs(0.0, q, lam, out)
+            ref = _adjoint(N, mesh, geom, lam)
+            d = (out - ref).astype(np.float64)
+            total += np.sum(d * d) / float(np.sum(ref * ref)) / 3
+        eng.close()
+        err[N] = np.sqrt(total)
+    print(" ".join("N %d: %.2e" % kv for kv in err.items()))
+    assert all(err[N] <= err[5] for N in range(1, 5))
