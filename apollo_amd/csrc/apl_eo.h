@@ -88,8 +88,9 @@ struct EoCfg {
   static constexpr int CV = 3 * Np * MH + 6 * MH + 16 * M;
   static constexpr int CF = 2 * Nfp * MH + 4 * MH + 24 * M + 2 * Np * MH;
   // face units [fb, fe) of wave w, in the order of the 3 NFU units
+  static_assert(W == 1 || W == 4 || W == 8, "the widths that the face units are split for");
   static constexpr int fb(int w) {
-    return W == 1 ? 0 : W == 2 ? (w == 0 ? 0 : 2 * NFU)
+    return W == 1 ? 0
          : W == 4 ? (w < 3 ? w : 3) * NFU
                   : (w < 6 ? (w >> 1) * NFU + (w & 1) * ((NFU + 1) / 2) : 3 * NFU);
   }
