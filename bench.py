@@ -54,17 +54,39 @@ def flop_alg(K, Np, Nc, Ng, m):
     return K * 2 * m * (3 * Nc * Np + 6 * Ng * Np)
 
 
-def flop_exec(linear, K, N, Np, Nc, Ng, m):
-    """Contraction flops the engine's kernel actually performs per RHS (no
-    padding): the cubature form does V_c (Nc Np), A_r|A_s (2 Nc Np), the face
-    traces (2 x 3 Ng (N+1)) and L (3 Ng Np) per variable; the nodal form of a
-    linear flux does Dt_r|Dt_s (2 Np^2) and Lt (3 (N+1) Np)."""
+AXIS_POINTS = (2, 5, 6, 6)    # cubature points of order 1..4 on the triangle's mirror axis
+
+
+def flop_exec(kernel, K, N, Np, Nc, Ng, m):
+    """Contraction flops `kernel` (kernel_name) performs per RHS, without its
+    padding.  Per variable, the cubature form takes V_c (Nc Np), A_r|A_s
+    (2 Nc Np), the face traces (2 x 3 Ng (N+1)) and L (3 Ng Np) products, the
+    nodal form of a linear flux Dt_r|Dt_s (2 Np^2) and Lt (3 (N+1) Np).  The
+    even-odd kernels take one row where those take two of mirrored points,
+    nodes or face points, but for L of the cubature form, and one correction
+    row."""
     Nfp = N + 1
-    if linear:
+    even = (Np + N // 2 + 1) // 2          # node pairs and nodes on the axis
+    if kernel.startswith("rhs_eo_linear_kernel"):
+        per = 2 * Np * even + (Nfp + (Nfp + 1) // 2) * Np
+    elif kernel.startswith("rhs_eo_kernel"):
+        ax = (AXIS_POINTS[N - 1] + 1) // 2
+        pairs = (Nc - AXIS_POINTS[N - 1]) // 2
+        per = 3 * Np * pairs + 2 * (even + Np) * ax + Np + 3 * Ng * (Nfp + Np)
+    elif "linear" in kernel:
         per = 2 * Np * Np + 3 * Nfp * Np
     else:
         per = 3 * Nc * Np + 6 * Ng * Nfp + 3 * Ng * Np
     return K * 2 * m * per
+
+
+def exec_peak(kernel, variant):
+    """The pipe a kernel's contractions run on and its peak: the matrix cores,
+    or the vector ALU, whose FP64 rate is theirs and whose FP32 rate without
+    packed instructions is its FP64 rate."""
+    if kernel.startswith(("rhs_kernel", "rhs_linear_kernel")):
+        return "mfma", PEAK["bf16" if variant.startswith("bf16") else variant[:4]]
+    return "valu", PEAK["fp64"]
 
 
 def bytes_alg_stage(K, Np, m):
@@ -131,15 +153,16 @@ def variant_figures(w, variant, r, steps):
     info = r["info"]
     K, N, Np, Nc, Ng, m = (info[k] for k in ("K", "N", "Np", "Nc", "Ng", "m"))
     lin = w.linear and VARIANTS[variant][1] in NODAL_ALGOS
+    kernel = kernel_name(w, variant)
     kern_s = r["gpu_ms"] * 1e-3 / (5 * steps)
     d = dict(dof_updates_per_s=K * Np * m / kern_s, ms_per_step=r["gpu_ms"] / steps,
              kernel_us=kern_s * 1e6, form="nodal" if lin else "cubature",
              tflops_alg=flop_alg(K, Np, Nc, Ng, m) / kern_s / 1e12,
-             tflops_exec=flop_exec(lin, K, N, Np, Nc, Ng, m) / kern_s / 1e12,
+             tflops_exec=flop_exec(kernel, K, N, Np, Nc, Ng, m) / kern_s / 1e12,
              gbs_alg=bytes_alg_stage(K, Np, m) / kern_s / 1e9)
     d["hbm_frac_alg"] = d["gbs_alg"] * 1e9 / PEAK["hbm"]
-    pk = PEAK["fp64" if variant.startswith("fp64") else ("fp32" if variant.startswith("fp32") else "bf16")]
-    d["mfma_frac_exec"] = d["tflops_exec"] * 1e12 / pk
+    pipe, pk = exec_peak(kernel, variant)
+    d[pipe + "_frac_exec"] = d["tflops_exec"] * 1e12 / pk
     return d
 
 
@@ -530,7 +553,7 @@ def main():
     # Roofline of the dominant kernel (the head variant's fused RHS + stage).
     # The nodal form executes ~2.5 flop per algorithmic byte, far below the
     # FP64 and FP32 ridges (9.8 and 19.7 flop/B), so its bound is HBM; the
-    # cubature form is reported against its MFMA peak beside it.
+    # cubature form is reported against its pipe's peak beside it.
     bpl = bytes_alg_stage(K, Np, m)
     lin = w.linear and VARIANTS[head][1] in NODAL_ALGOS
     kname = kernel_name(w, head)
@@ -543,9 +566,9 @@ def main():
                                       % (5 * args.steps),
                             "bytes_per_launch": bpl}
     else:
-        pk = PEAK["fp64" if head.startswith("fp64") else "fp32"]
+        pipe, pk = exec_peak(kname, head)
         ach = h["tflops_alg"] * 1e12
-        line["roofline"] = {"bound": "mfma", "achieved": ach / 1e12, "peak": pk / 1e12,
+        line["roofline"] = {"bound": pipe, "achieved": ach / 1e12, "peak": pk / 1e12,
                             "unit": "TFLOP/s", "frac": ach / pk, "traffic": None,
                             "kernel": kname + " (fused RHS + LSERK4 stage), avg over %d launches"
                                       % (5 * args.steps),
@@ -561,9 +584,9 @@ def main():
                 "unit": "GB/s", "frac": out[v]["hbm_frac_alg"],
                 "traffic": measured_traffic("tm_cavity_256_N5/%s" % v), "kernel": kernel_name(w, v)}
         else:
-            pk = PEAK["fp64" if v.startswith("fp64") else ("fp32" if v.startswith("fp32") else "bf16")]
+            pipe, pk = exec_peak(kernel_name(w, v), v)
             line["roofline_variants"][v] = {
-                "bound": "mfma", "achieved_exec": out[v]["tflops_exec"], "peak": pk / 1e12,
+                "bound": pipe, "achieved_exec": out[v]["tflops_exec"], "peak": pk / 1e12,
                 "unit": "TFLOP/s", "frac": out[v]["tflops_exec"] * 1e12 / pk,
                 "traffic": measured_traffic("tm_cavity_256_N5/%s" % v), "kernel": kernel_name(w, v)}
     if "fp32" in out and "fp64" in out:
