@@ -163,10 +163,8 @@ static int dev_alloc(apl_handle *h, void **dst, size_t bytes) {
 // The cubature form in FP32 at N <= 3 runs on the VALU kernel unless
 // APL_ALGO_CUBATURE_MFMA asks for the MFMA kernel: measured faster on the 2D
 // Euler vortex at N = 3 (us per fused stage, VALU vs MFMA): K = 8192 15.4 vs
-// 16.8; K = 131072 67.7 vs 75.2.  In FP64 it runs on the even-odd kernel up
-// to this order: N = 3, K = 131072 68 us against 92 on the VALU kernel's FP64
-// form that it replaced, N = 4, K = 524288 404 against 585 on MFMA.
-constexpr int EO_MAX_ORDER = 4;
+// 16.8; K = 131072 67.7 vs 75.2.  In FP64 it runs on the even-odd kernel where
+// eo_order() says so.
 constexpr bool VALU_BY_DEFAULT = true;
 // The nodal form of MAXWELL_TM3 runs on the VALU kernel under
 // APL_ALGO_AUTO (FP64 and FP32).
@@ -1049,7 +1047,7 @@ int apl_create(const apl_mesh *mesh, const apl_params *params, apl_handle **out)
   h->eo = params->precision == APL_PREC_FP64 &&
           (h->linear ? params->algorithm == APL_ALGO_AUTO && !h->valu &&
                            eo_linear_takes(params->eqn, params->order, mesh->K)
-                     : params->order <= EO_MAX_ORDER && params->algorithm != APL_ALGO_CUBATURE_MFMA);
+                     : eo_order(params->order, M) && params->algorithm != APL_ALGO_CUBATURE_MFMA);
   h->K = mesh->K;
   h->M = M;
   h->Nv = mesh->Nv;

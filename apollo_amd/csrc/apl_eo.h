@@ -69,6 +69,14 @@ struct EoNodes {
   }
 };
 
+// Orders and variable counts whose FP64 cubature form runs here (us per stage:
+// Euler N = 3, K = 131072 68 against 92 on the vector-ALU kernel's FP64 form that
+// this kernel replaced; N = 4, K = 524288 404 against 585 on MFMA).  A lane holds
+// the state and the residual of half the variables, and the 8-variable system at
+// N = 4 spills 400-530 bytes: 4 LSERK4 steps (20 stages), here / on MFMA, K = 3200
+// 752 / 706 us, K = 8192 909 / 727, K = 51200 5205 / 2677.
+constexpr bool eo_order(int N, int M) { return N <= 3 || (N == 4 && M <= 5); }
+
 template <int N, int EQN, int W_>
 struct EoCfg {
   using O = Order<N>;

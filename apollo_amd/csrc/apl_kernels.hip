@@ -56,7 +56,7 @@ static int launch_eo_linear(hipStream_t s, const RhsArgs &a) {
 // kind: 0 the cubature form on MFMA, 1 the nodal form (linear fluxes) on
 // MFMA, 2 the cubature form on the VALU kernel (N <= 3, FP32), 3 the nodal
 // form on the VALU kernel (TM, FP64 and FP32), 4 the cubature form on the
-// even-odd kernel (N <= 4, FP64), 5 the nodal form on the even-odd kernel
+// even-odd kernel (FP64, eo_order), 5 the nodal form on the even-odd kernel
 // (FP64)
 template <int N, int EQN, int FLUX, typename T>
 static int launch_typed(int kind, hipStream_t s, const RhsArgs &a, int nblocks) {
@@ -98,7 +98,7 @@ static int launch_typed(int kind, hipStream_t s, const RhsArgs &a, int nblocks) 
   }
   if (kind == 1 || kind == 3) return APL_ERR_ARG;
   if (kind == 4) {
-    if constexpr (N <= 4 && sizeof(T) == 8) {
+    if constexpr (eo_order(N, Vars<EQN>::M) && sizeof(T) == 8) {
       if constexpr (EQN == APL_EQN_EULER5 || EQN == APL_EQN_EULER4)
         if (a.vortex) return launch_eo<N, EQN, FLUX, 4, true>(s, a);
       // One wave per group once the waves fill the card's 1024 SIMDs twice

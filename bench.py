@@ -458,8 +458,8 @@ def calibrate_copy(mib, reps=10):
 def kernel_name(w, variant):
     """The engine's kernel for a variant: the nodal kernel for linear fluxes
     (algorithm 0; in FP64 the even-odd one for the 8-variable system and small
-    TM meshes), the even-odd cubature kernel in FP64 at N <= 4, the vector-ALU
-    one in FP32 at N <= 3 (algorithms 0, 1, 3; eight waves per group below 512
+    TM meshes), the even-odd cubature kernel in FP64 at N <= 4 (8 variables:
+    N <= 3), the vector-ALU one in FP32 at N <= 3 (algorithms 0, 1, 3; eight waves per group below 512
     groups), else the MFMA cubature kernel."""
     N = w.order
     prec, algo = VARIANTS[variant]
@@ -471,7 +471,7 @@ def kernel_name(w, variant):
         return "rhs_eo_linear_kernel<%d,%d,%d>" % (N, w.eqn, w.flux)
     if w.linear and algo in NODAL_ALGOS:
         return "rhs_linear_kernel<%d,%d,%d,%s>" % (N, w.eqn, w.flux, ty)
-    if N <= 4 and prec == 0 and algo != 2:
+    if N <= (3 if w.m == 8 else 4) and prec == 0 and algo != 2:
         return "rhs_eo_kernel<%d,%d,%d>" % (N, w.eqn, w.flux)
     if N <= 3 and prec == 1 and algo != 2:
         nw = 8 if (w.K + 63) // 64 < 512 else 4

@@ -95,7 +95,8 @@ enum apl_algorithm {
                               8-variable system and for TM meshes of at most
                               8192 elements (4096 at N = 8), else on MFMA.  The
                               cubature form runs on the vector ALU at N <= 4
-                              in FP64 and N <= 3 in FP32, on MFMA otherwise  */
+                              (8 variables: N <= 3) in FP64 and N <= 3 in
+                              FP32, on MFMA otherwise                        */
   APL_ALGO_CUBATURE = 1,   /* always Apollo's over-integrated cubature form
                               (wxcubature2d.cc:288-382), on the kernels
                               APL_ALGO_AUTO picks for it                     */

@@ -63,6 +63,22 @@ def test_eo_boundaries(N):
         _check(case, case.state())
 
 
+@pytest.mark.parametrize("n", [3, 4, 65])
+@pytest.mark.parametrize("N", [3, 4])
+def test_eo_eight_variables(N, n):
+    """The last order of the 8-variable system on this kernel and the first
+    that the MFMA kernel takes (the same bits as when it is asked for)."""
+    case = maxwell_case(n=n, N=N, m=8, bc=E.BC_PEC)
+    q = case.state()
+    _check(case, q)
+    out = [np.zeros_like(q), np.zeros_like(q)]
+    for o, algorithm in zip(out, (E.ALGO_CUBATURE, E.ALGO_CUBATURE_MFMA)):
+        eng = _engine(case, algorithm)
+        eng.rhs(0.0, q, o)
+        eng.close()
+    assert np.array_equal(out[0], out[1]) == (N == 4)
+
+
 @pytest.mark.parametrize("N,n", [(2, 5), (3, 65), (4, 20)])
 def test_eo_steppers(N, n):
     case = euler_case(n=n, N=N, m=4)
