@@ -478,6 +478,18 @@ struct AdjGroup {
   static constexpr int W = group_waves(AdjLds<N, EQN>::doubles, 4 * AdjWaves<N, EQN>::value);
 };
 
+// Whether the neighbours' face nodes are gathered after the state is staged,
+// two items in flight, instead of with it: where the values held meanwhile cost
+// more registers than their latency is worth (us, with the state / after it,
+// J^T at K = 20000 if not said otherwise: 5 variables N = 7 427 / 374, N = 6
+// reverse stage 216 / 191, N = 5 126 / 127; 4 variables N = 7 304 / 274, N = 6
+// 133 / 134; TM N = 8 186 / 190; 8 variables, K = 2738, N = 7 140.7 / 138.7, N = 8
+// 211 / 207, N = 6 69.6 / 70.1).
+template <int N, int EQN>
+struct AdjGather {
+  static constexpr bool late = EQN != APL_EQN_MAXWELL_TM3 && N >= (EQN == APL_EQN_EULER5 ? 6 : 7);
+};
+
 // STAGE: the reverse-LSERK4 stage kernel (mode 1: lam = rbar + b qbar, the
 // stage update and the next stage's face weights); otherwise out = J^T lam
 // (mode 0).
@@ -515,16 +527,19 @@ __global__ void __launch_bounds__((64 * AdjGroup<N, EQN>::W), (AdjWaves<N, EQN>:
   // (as in rhs_kernel)
   const int code0 = a.fcode[ge * 3], code1 = a.fcode[ge * 3 + 1], code2 = a.fcode[ge * 3 + 2];
   constexpr int NGI = (3 * Nfp + 3) / 4, NI1 = (L::I1D + 63) / 64;
-  double i1v[NI1], nbv[NGI][M];
+  constexpr bool LATE = AdjGather<N, EQN>::late;
+  double i1v[NI1], nbv[LATE ? 1 : NGI][M];
 #pragma unroll
   for (int j = 0; j < NI1; ++j) i1v[j] = a.I1D[min(lane + 64 * j, L::I1D - 1)];
   StageBuf<ES> buf;
   stage_load<ES>(buf, a.q + e0 * ES, cnt, lane);
   __builtin_amdgcn_sched_barrier(0);
+  if constexpr (!LATE) {
 #pragma unroll
-  for (int j = 0; j < NGI; ++j)
-    gather_face_node<N, M>(a.q, 4 * j + lg, code0, code1, code2, ge, nbv[j]);
-  __builtin_amdgcn_sched_barrier(0);
+    for (int j = 0; j < NGI; ++j)
+      gather_face_node<N, M>(a.q, 4 * j + lg, code0, code1, code2, ge, nbv[j]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   stage_store<ES, 16>(XT, buf, a.q + e0 * ES, cnt, lane);
   if constexpr (STAGE)
     axpy_stage_transposed<ES>(LT, a.lam + e0 * ES, a.qbar + e0 * ES, a.rk_b, cnt, lane);
@@ -534,12 +549,14 @@ __global__ void __launch_bounds__((64 * AdjGroup<N, EQN>::W), (AdjWaves<N, EQN>:
 #pragma unroll
   for (int j = 0; j < NI1; ++j)
     if (64 * (j + 1) <= L::I1D || lane + 64 * j < L::I1D) I1[lane + 64 * j] = i1v[j];
-#pragma unroll
+  if constexpr (LATE) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll(LATE ? 2 : NGI)
   for (int j = 0; j < NGI; ++j) {
-    const int k = 4 * j + lg;
+    const int k = 4 * j + lg, jv = LATE ? 0 : j;
+    if constexpr (LATE) gather_face_node<N, M>(a.q, k, code0, code1, code2, ge, nbv[jv]);
     if (4 * j + 4 <= 3 * Nfp || k < 3 * Nfp) {
 #pragma unroll
-      for (int v = 0; v < M; ++v) PT[(k * M + v) * 16 + el] = nbv[j][v];
+      for (int v = 0; v < M; ++v) PT[(k * M + v) * 16 + el] = nbv[jv][v];
     }
   }
   wave_sync();
