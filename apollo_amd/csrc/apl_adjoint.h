@@ -573,11 +573,25 @@ __global__ void __launch_bounds__((64 * AdjGroup<N, EQN>::W), (AdjWaves<N, EQN>:
     V4 qc[M], fr[M], fs[M];
 #pragma unroll
     for (int v = 0; v < M; ++v) qc[v] = fr[v] = fs[v] = V4{0, 0, 0, 0};
+    // The operator rows of the first AHEAD steps requested before the first
+    // product, where the compiler alone requests two steps' (TM N = 8 reverse
+    // stage, the other kernels' five and more: K = 20000 281 -> 220 us).
+    constexpr int AHEAD = STAGE && N == 8 && M == 3 ? 5 : 0;
+    double pv[AHEAD + 1], pr[AHEAD + 1], ps[AHEAD + 1];
+    if constexpr (AHEAD > 0) {
+#pragma unroll
+      for (int ks = 0; ks < AHEAD; ++ks) {
+        pv[ks] = a.Avc[(cc * NKS1 + ks) * 64 + lane];
+        pr[ks] = a.Aart[(cc * NKS1 + ks) * 64 + lane];
+        ps[ks] = a.Aast[(cc * NKS1 + ks) * 64 + lane];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
     for (int ks = 0; ks < NKS1; ++ks) {
-      const double a1 = a.Avc[(cc * NKS1 + ks) * 64 + lane];
-      const double ar = a.Aart[(cc * NKS1 + ks) * 64 + lane];
-      const double as = a.Aast[(cc * NKS1 + ks) * 64 + lane];
+      const double a1 = ks < AHEAD ? pv[ks] : a.Avc[(cc * NKS1 + ks) * 64 + lane];
+      const double ar = ks < AHEAD ? pr[ks] : a.Aart[(cc * NKS1 + ks) * 64 + lane];
+      const double as = ks < AHEAD ? ps[ks] : a.Aast[(cc * NKS1 + ks) * 64 + lane];
 #pragma unroll
       for (int v = 0; v < M; ++v) {
         const double bx = XT[((4 * ks + lg) * M + v) * 16 + el];
