@@ -90,6 +90,21 @@ constexpr int VALU_WAVES = 3;
 template <typename S>
 using cptr_t = const __attribute__((address_space(4))) S *;
 
+// The kernel's arguments read again from the argument segment, past what the
+// compiler holds of them: it loads every argument at the kernel's start, and
+// those of the epilogue crowd the operators' scalar registers out (N = 1: 66
+// writes of scalars to vector lanes and 278 reads back; us per launch, held /
+// read again: 4 variables N = 1, K = 320 7.4 / 6.6, K = 32768 9.1 / 8.4, 5
+// variables N = 2, K = 80000 31.6 / 30.6).
+__device__ __forceinline__ RhsArgs late_args() {
+  typedef const __attribute__((address_space(4))) char *seg_t;
+  seg_t k = (seg_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(k));
+  RhsArgs r;
+  __builtin_memcpy(&r, __builtin_assume_aligned((const char *)k, 16), sizeof(r));
+  return r;
+}
+
 template <int N, int EQN, int FLUX, typename S, int W>
 __global__ void __launch_bounds__(64 * W, VALU_WAVES)
     rhs_valu_kernel(RhsArgs a) {
@@ -340,6 +355,7 @@ __global__ void __launch_bounds__(64 * W, VALU_WAVES)
     }
     if (h > 1) __syncthreads();
   }
+  const RhsArgs al = late_args();
   if (wave == 0) {
     // wave 0's reads of RED are all issued before its first write of OUT,
     // which overlaps them; one wave's LDS operations complete in order
@@ -353,9 +369,9 @@ __global__ void __launch_bounds__(64 * W, VALU_WAVES)
 
   // 5. wave w < 4 writes elements [16 w, 16 w + 16) of the group
   const long eb = e0 + 16 * wave;
-  if (wave < 4 && eb < a.K) {
-    const int cw = (int)min((long)16, (long)a.K - eb);
-    ef |= write_batch<ES>(a, OUT + 16 * wave * ES, eb, cw, lane);
+  if (wave < 4 && eb < al.K) {
+    const int cw = (int)min((long)16, (long)al.K - eb);
+    ef |= write_batch<ES>(al, OUT + 16 * wave * ES, eb, cw, lane);
   }
   for (int off = 32; off > 0; off >>= 1) {
     const double o = __shfl_xor(lmax, off);
@@ -367,7 +383,7 @@ __global__ void __launch_bounds__(64 * W, VALU_WAVES)
     EFW[wave] = ef;
   }
   __syncthreads();
-  if (lane == 0 && wave < 4 && eb < a.K) {
+  if (lane == 0 && wave < 4 && eb < al.K) {
     double m = SPD[0];
     unsigned e = EFW[0];
 #pragma unroll
@@ -375,8 +391,8 @@ __global__ void __launch_bounds__(64 * W, VALU_WAVES)
       m = SPD[w] > m ? SPD[w] : m;
       e |= EFW[w];
     }
-    if (a.speed_part) a.speed_part[grp * 4 + wave] = m;
-    if (wave == 0 && e) atomicOr(a.err, e);
+    if (al.speed_part) al.speed_part[grp * 4 + wave] = m;
+    if (wave == 0 && e) atomicOr(al.err, e);
   }
 }
 
