@@ -120,11 +120,13 @@ struct EoCfg {
   static constexpr int LDS = 32 * ESP + RED + W + (W + 1) / 2;
 };
 
-// Waves per SIMD asked of the register allocator.
+// Waves per SIMD asked of the register allocator: three where 168 registers
+// hold a lane's state and residual.  The 5- and 8-variable systems at N = 2 spill
+// 64-190 bytes there (4 LSERK4 steps, three / two waves: 5 variables HLL, K =
+// 12800 350 / 310 us, K = 131072 1506 / 1341; 8 variables, K = 20000 576 / 411).
 template <int N, int EQN, int W>
 struct EoWaves {
-  static constexpr int NR = Order<N>::Np * ((Vars<EQN>::M + 1) / 2);   // doubles of R per lane
-  static constexpr int value = NR <= 24 && W < 8 ? 3 : 2;
+  static constexpr int value = W < 8 && (N == 1 || (N <= 3 && Vars<EQN>::M <= 4)) ? 3 : 2;
 };
 
 // Exchange lanes 32..63 of x with lanes 0..31 of y.

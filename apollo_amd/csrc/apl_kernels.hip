@@ -106,12 +106,19 @@ static int launch_typed(int kind, hipStream_t s, const RhsArgs &a, int nblocks) 
       // 16384 groups 404 / 494; 5-variable N = 4, 4096 groups 162 / 240);
       // below that the last round of long waves costs more than the split
       // (N = 3, 4096 groups 74 / 67; N = 4, 2500 groups 96 / 78), unless a
-      // CU's LDS holds only one four-wave group.  Eight
-      // while a CU gets at most one group (256 groups, N = 4: 15.4 / 16.4
-      // with four).
+      // CU's LDS holds only one four-wave group.  At N = 1 and, with five
+      // variables or more, N = 2 the waves are short and the reduction is more of
+      // a group's work: one from 1536 groups on (N = 1: TM, 3906 groups 21.7 /
+      // 27.1, Euler, 1600 17.0 / 18.0; N = 2, 5 variables HLL, 1600 groups 35.7 /
+      // 38.1, 1156 33.3 / 29.1), for eight variables at N = 1 from 1024 on (16.8 /
+      // 18.2).  Eight while a CU gets at most one group (256 groups, N = 4: 15.4 /
+      // 16.4 with four).
       const int groups = (a.K + 31) / 32;
       constexpr bool PAIR = 2 * EoCfg<N, EQN, 4>::LDS * 8 <= 163840;
-      if (groups >= (PAIR ? 2 * EoWaves<N, EQN, 1>::value : 1) * 1024) return launch_eo<N, EQN, FLUX, 1>(s, a);
+      constexpr int M = Vars<EQN>::M;
+      constexpr int ONE = N == 1 && M == 8 ? 1024 : N == 1 || (N == 2 && M >= 5) ? 1536
+                          : (PAIR ? 2 * EoWaves<N, EQN, 1>::value : 1) * 1024;
+      if (groups >= ONE) return launch_eo<N, EQN, FLUX, 1>(s, a);
       if constexpr (EoCfg<N, EQN, 8>::LDS * 8 <= 163840)
         if (groups <= 256) return launch_eo<N, EQN, FLUX, 8>(s, a);
       return launch_eo<N, EQN, FLUX, 4>(s, a);

@@ -79,6 +79,18 @@ def test_eo_eight_variables(N, n):
     assert np.array_equal(out[0], out[1]) == (N == 4)
 
 
+@pytest.mark.parametrize("N,m,n", [(1, 4, 156), (1, 4, 157), (2, 5, 157), (1, 8, 128), (2, 8, 157)])
+def test_eo_one_wave_groups_small_orders(N, m, n):
+    """One-wave groups from 1536 groups on (K = 49152; n = 156 and 157 lie on
+    either side), for eight variables at N = 1 from 1024 on."""
+    if m == 8:
+        case = maxwell_case(n=n, N=N, m=m, bc=E.BC_PEC)
+        _check(case, case.state())
+    else:
+        case = euler_case(n=n, N=N, m=m)
+        _check(case, case.state(amp=1e-3))
+
+
 @pytest.mark.parametrize("N,n", [(2, 5), (3, 65), (4, 20)])
 def test_eo_steppers(N, n):
     case = euler_case(n=n, N=N, m=4)
