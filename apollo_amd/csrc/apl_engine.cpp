@@ -40,7 +40,7 @@ struct apl_handle_s {
   apl_params params;
   int K = 0, M = 0, Nv = 0;
   bool linear = false;   // nodal linear-flux kernel (Maxwell, APL_ALGO_AUTO)
-  bool valu = false;     // VALU kernel: cubature form (N <= 3, FP32) or nodal form
+  bool valu = false;     // VALU kernel: cubature form (N <= 3, FP32; TM, FP64) or nodal form
   bool eo = false;       // on an even-odd kernel (FP64): rhs_eo_kernel, or rhs_eo_linear_kernel if linear
   Operators ops;
   Geometry geo;
@@ -367,7 +367,7 @@ static void make_fragments(const Operators &o, std::vector<T> &A1, std::vector<T
       }
 }
 
-// Point tables of the VALU cubature kernel (apl_valu.h, FP32): row c of A1 holds
+// Point tables of the VALU cubature kernel (apl_valu.h): row c of A1 holds
 // V_c[c, 0..Np), A_r[0..Np, c), A_s[0..Np, c); row k of A3 holds -L[0..Np, k).
 template <typename T>
 static void make_valu_tables(const Operators &o, std::vector<T> &A1, std::vector<T> &A3) {
@@ -1041,11 +1041,13 @@ int apl_create(const apl_mesh *mesh, const apl_params *params, apl_handle **out)
               (params->algorithm == APL_ALGO_AUTO && NODAL_VALU_BY_DEFAULT &&
                params->eqn == APL_EQN_MAXWELL_TM3 && params->precision != APL_PREC_BF16X3);
   else
-    h->valu = params->order <= 3 && params->precision == APL_PREC_FP32_MFMA &&
-              (params->algorithm == APL_ALGO_CUBATURE_VALU ||
-               (params->algorithm != APL_ALGO_CUBATURE_MFMA && VALU_BY_DEFAULT));
-  h->eo = params->precision == APL_PREC_FP64 &&
-          (h->linear ? params->algorithm == APL_ALGO_AUTO && !h->valu &&
+    h->valu = params->precision == APL_PREC_FP32_MFMA
+                  ? params->order <= 3 && (params->algorithm == APL_ALGO_CUBATURE_VALU ||
+                                           (params->algorithm != APL_ALGO_CUBATURE_MFMA && VALU_BY_DEFAULT))
+                  : params->precision == APL_PREC_FP64 && params->algorithm != APL_ALGO_CUBATURE_MFMA &&
+                        valu_takes_fp64(params->eqn, params->order, mesh->K);
+  h->eo = params->precision == APL_PREC_FP64 && !h->valu &&
+          (h->linear ? params->algorithm == APL_ALGO_AUTO &&
                            eo_linear_takes(params->eqn, params->order, mesh->K)
                      : eo_order(params->order, M) && params->algorithm != APL_ALGO_CUBATURE_MFMA);
   h->K = mesh->K;

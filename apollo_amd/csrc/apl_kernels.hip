@@ -32,6 +32,16 @@ static int launch_batches(K kern, hipStream_t s, const A &a, int nbatches) {
   return hipGetLastError() == hipSuccess ? APL_OK : APL_ERR_HIP;
 }
 
+// The vector-ALU cubature kernel: groups of 64 elements, W waves each.
+template <int N, int EQN, int FLUX, typename T, int W>
+static int launch_valu(hipStream_t s, const RhsArgs &a) {
+  auto kern = rhs_valu_kernel<N, EQN, FLUX, T, W>;
+  const size_t lds = sizeof(double) * (size_t)ValuLds<N, EQN, T, W>::doubles;
+  if (!allow_lds(kern, lds)) return APL_ERR_UNSUPPORTED;
+  hipLaunchKernelGGL(kern, dim3((a.K + 63) / 64), dim3(64 * W), lds, s, a);
+  return hipGetLastError() == hipSuccess ? APL_OK : APL_ERR_HIP;
+}
+
 // The even-odd kernel: groups of 32 elements, W waves each.
 template <int N, int EQN, int FLUX, int W, bool VTX = false>
 static int launch_eo(hipStream_t s, const RhsArgs &a) {
@@ -127,21 +137,13 @@ static int launch_typed(int kind, hipStream_t s, const RhsArgs &a, int nblocks) 
     }
   }
   if (kind == 2) {
-    if constexpr (N <= 3 && sizeof(T) == 4) {
+    if constexpr (N <= 3 && (sizeof(T) == 4 || (sizeof(T) == 8 && valu_fp64_order(EQN, N)))) {
       // 64 elements per workgroup of four waves, or of eight on small meshes
       const int groups = (a.K + 63) / 64;
-      if (groups < VALU_SMALL_GROUPS && ValuLds<N, EQN, T, 8>::doubles * 8 <= 163840) {
-        auto kern = rhs_valu_kernel<N, EQN, FLUX, T, 8>;
-        const size_t lds = sizeof(double) * (size_t)ValuLds<N, EQN, T, 8>::doubles;
-        if (!allow_lds(kern, lds)) return APL_ERR_UNSUPPORTED;
-        hipLaunchKernelGGL(kern, dim3(groups), dim3(512), lds, s, a);
-      } else {
-        auto kern = rhs_valu_kernel<N, EQN, FLUX, T, 4>;
-        const size_t lds = sizeof(double) * (size_t)ValuLds<N, EQN, T, 4>::doubles;
-        if (!allow_lds(kern, lds)) return APL_ERR_UNSUPPORTED;
-        hipLaunchKernelGGL(kern, dim3(groups), dim3(256), lds, s, a);
-      }
-      return hipGetLastError() == hipSuccess ? APL_OK : APL_ERR_HIP;
+      if constexpr (sizeof(T) == 4)
+        if (groups < VALU_SMALL_GROUPS && ValuLds<N, EQN, T, 8>::doubles * 8 <= 163840)
+          return launch_valu<N, EQN, FLUX, T, 8>(s, a);
+      return launch_valu<N, EQN, FLUX, T, 4>(s, a);
     } else {
       return APL_ERR_UNSUPPORTED;
     }

@@ -1,5 +1,6 @@
 // apl_valu.h -- the cubature-form RHS in FP32 on the vector ALU for N <= 3
-// (gfx950); FP64 runs on the even-odd kernel (apl_eo.h).
+// (gfx950); FP64 runs on the even-odd kernel (apl_eo.h) but for the TM meshes
+// of valu_takes_fp64().
 //
 // The same RHS as rhs_kernel (apl_device.h), Apollo's over-integrated
 // cubature form (src/subsolvers/wxnodaldg2dmethod.cc:320-510,
@@ -85,7 +86,22 @@ struct ValuLds {
 constexpr int VALU_SMALL_GROUPS = 512;
 
 // waves per SIMD asked of the register allocator
-constexpr int VALU_WAVES = 3;
+template <typename S>
+struct ValuWaves {
+  static constexpr int value = sizeof(S) == 8 ? 2 : 3;
+};
+
+// TM meshes whose FP64 cubature form runs here: one lane per element, where the
+// even-odd kernel's groups start a second round on the card and its waves' few
+// points do not pay for sharing them (us per 4 LSERK4 steps, here / there with
+// four waves / one: N = 1, K = 33282 237 / 259 / 258, 41472 244 / 287 / 267, 51200
+// 284 / 312 / 275; N = 2, K = 41472 331 / 368 / 383, 125000 639 / 709 / 650, 320000
+// 1193 / 1437 / 1313, 460800 1874 / - / 1767; at K = 32768 the four waves' groups
+// are one round, N = 1 230 / 227).
+constexpr bool valu_fp64_order(int eqn, int N) { return eqn == APL_EQN_MAXWELL_TM3 && N <= 2; }
+constexpr bool valu_takes_fp64(int eqn, int N, int K) {
+  return valu_fp64_order(eqn, N) && K > 32768 && K < (N == 1 ? 49152 : 442368);
+}
 
 template <typename S>
 using cptr_t = const __attribute__((address_space(4))) S *;
@@ -106,7 +122,7 @@ __device__ __forceinline__ RhsArgs late_args() {
 }
 
 template <int N, int EQN, int FLUX, typename S, int W>
-__global__ void __launch_bounds__(64 * W, VALU_WAVES)
+__global__ void __launch_bounds__(64 * W, ValuWaves<S>::value)
     rhs_valu_kernel(RhsArgs a) {
   using C = ValuCfg<N, EQN, W>;
   using L = ValuLds<N, EQN, S, W>;
@@ -114,8 +130,7 @@ __global__ void __launch_bounds__(64 * W, VALU_WAVES)
   constexpr int ES = C::ES, ESP = C::ESP, VW = C::VW, FW = C::FW, NFG = C::NFG;
   constexpr int NT = 64 * W;   // threads
   // FP32 face traces and flux where the FP32 MFMA kernel uses them
-  static_assert(sizeof(S) == 4, "FP64 runs on the even-odd kernel");
-  constexpr bool F32 = FLUX == APL_FLUX_LF &&
+  constexpr bool F32 = sizeof(S) == 4 && FLUX == APL_FLUX_LF &&
                        (EQN == APL_EQN_EULER5 || EQN == APL_EQN_EULER4);
   typedef typename std::conditional<F32, float, double>::type TR;   // trace type
 

@@ -459,8 +459,9 @@ def kernel_name(w, variant):
     """The engine's kernel for a variant: the nodal kernel for linear fluxes
     (algorithm 0; in FP64 the even-odd one for the 8-variable system and small
     TM meshes), the even-odd cubature kernel in FP64 at N <= 4 (8 variables:
-    N <= 3), the vector-ALU one in FP32 at N <= 3 (algorithms 0, 1, 3; eight waves per group below 512
-    groups), else the MFMA cubature kernel."""
+    N <= 3), the vector-ALU one in FP64 for TM meshes of more than 32768 elements
+    at N <= 2 (up to a size) and in FP32 at N <= 3 (algorithms 0, 1, 3; eight
+    waves per group below 512 groups), else the MFMA cubature kernel."""
     N = w.order
     prec, algo = VARIANTS[variant]
     ty = {"fp64": "double", "fp32": "float", "bf16x3": "apl::Bf16x3"}[variant.split("_")[0]]
@@ -471,6 +472,8 @@ def kernel_name(w, variant):
         return "rhs_eo_linear_kernel<%d,%d,%d>" % (N, w.eqn, w.flux)
     if w.linear and algo in NODAL_ALGOS:
         return "rhs_linear_kernel<%d,%d,%d,%s>" % (N, w.eqn, w.flux, ty)
+    if w.m == 3 and N <= 2 and prec == 0 and algo != 2 and 32768 < w.K < (49152 if N == 1 else 442368):
+        return "rhs_valu_kernel<%d,%d,%d,%s,4>" % (N, w.eqn, w.flux, ty)
     if N <= (3 if w.m == 8 else 4) and prec == 0 and algo != 2:
         return "rhs_eo_kernel<%d,%d,%d>" % (N, w.eqn, w.flux)
     if N <= 3 and prec == 1 and algo != 2:

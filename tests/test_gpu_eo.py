@@ -91,6 +91,25 @@ def test_eo_one_wave_groups_small_orders(N, m, n):
         _check(case, case.state(amp=1e-3))
 
 
+@pytest.mark.parametrize("flux", [E.FLUX_UPWIND, E.FLUX_LF])
+@pytest.mark.parametrize("N,n", [(1, 128), (1, 129), (1, 157), (2, 129)])
+def test_eo_tm_meshes(N, n, flux):
+    """TM meshes at the limits of the vector-ALU kernel's FP64 form, between
+    K = 32768 (the last four-wave mesh here) and, at N = 1, 49152 (one-wave
+    groups from there); PEC walls, a partial last group but for n = 128."""
+    case = maxwell_case(n=n, N=N, m=3, bc=E.BC_PEC, flux=flux)
+    q = case.state()
+    _check(case, q)
+    eng = _engine(case)
+    got = q.copy()
+    eng.lserk4(0.0, 1e-4, 1, got)
+    eng.close()
+    with O.exact_geometry():
+        ref = from_oracle(case.params.eqn, O.lserk4(case.omesh, case.ophys, 0.0, 1e-4, 1,
+                                                    to_oracle(case.params.eqn, q)))
+    assert rel_l2(got - q, ref - q) <= 1e-11
+
+
 @pytest.mark.parametrize("N,n", [(2, 5), (3, 65), (4, 20)])
 def test_eo_steppers(N, n):
     case = euler_case(n=n, N=N, m=4)
