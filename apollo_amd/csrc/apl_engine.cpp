@@ -1450,6 +1450,11 @@ int apl_rhs_noalloc(apl_handle *h, double t, const double *q, double *rhs, doubl
   return APL_OK;
 }
 
+// A device state of at most this many nodes is copied to the host and its wave
+// speed taken there (us a call, 5 variables, host / kernel and report: 864 nodes
+// 20 / 39, 1728 28 / 40, 3888 48 / 40).
+constexpr size_t INITIAL_DT_HOST_NODES = 2048;
+
 int apl_initial_dt(apl_handle *h, const double *q, double cfl, double *dt, int where) {
   if (!h || !q || !dt) return APL_ERR_ARG;
   // Roe speeds of the node state against itself (wxnodaldg2dmethod.cc:201-213,
@@ -1460,7 +1465,7 @@ int apl_initial_dt(apl_handle *h, const double *q, double cfl, double *dt, int w
   double maxSpeed = 0.0;
   if (p.eqn != APL_EQN_EULER5 && p.eqn != APL_EQN_EULER4) {
     maxSpeed = std::max(std::max(p.chi * p.c0, p.gamma_ph * p.c0), p.c0);
-  } else if (where == APL_DEVICE) {
+  } else if (where == APL_DEVICE && nodes > INITIAL_DT_HOST_NODES) {
     // A synchronous copy waits for every blocking stream, on any of which the
     // caller may have filled q; the handle's stream alone waits for the null
     // stream's work, or where it is the caller's for its own.
@@ -1474,8 +1479,14 @@ int apl_initial_dt(apl_handle *h, const double *q, double cfl, double *dt, int w
     if ((rc = begin_flags(h)) || (rc = report(h, h->d_speed, n, &s2))) return rc;
     maxSpeed = std::sqrt(s2);
   } else {
+    std::vector<double> hq;
+    if (where == APL_DEVICE) {
+      hq.resize(nodes * M);
+      HIPCHK(h, hipMemcpy(hq.data(), q, sizeof(double) * hq.size(), hipMemcpyDeviceToHost));
+    }
+    const double *src = where == APL_DEVICE ? hq.data() : q;
     for (size_t i = 0; i < nodes; ++i) {
-      const double *d = q + i * M;
+      const double *d = src + i * M;
       const double rho = d[0], mu = d[1], mv = d[2];
       const double mw = (p.eqn == APL_EQN_EULER5) ? d[3] : 0.0;
       const double E = (p.eqn == APL_EQN_EULER5) ? d[4] : d[3];

@@ -1,5 +1,6 @@
 """initial_dt of a state that another blocking stream is still writing: the
-call waits for it, on a handle with its own stream and on the null stream."""
+call waits for it, on a handle with its own stream and on the null stream; and
+of states on either side of the size up to which the host computes it."""
 import ctypes
 import re
 
@@ -40,3 +41,17 @@ def test_initial_dt_waits_for_blocking_streams(null_stream):
     assert dt != eng.initial_dt(before, 0.5)
     eng.close()
     assert hip.hipStreamDestroy(raw) == 0
+
+
+@pytest.mark.parametrize("m", [4, 5])
+@pytest.mark.parametrize("n,N", [(1, 1), (13, 2), (14, 2), (18, 2), (19, 2)])
+def test_initial_dt_host_and_device_states(n, N, m):
+    """2028 nodes are the last below the limit of 2048 here, 2352 the first above."""
+    torch = pytest.importorskip("torch")
+    case = euler_case(n=n, N=N, m=m, periodic=False)
+    q = case.state(amp=1e-3, seed=n)
+    eng = E.Engine(case.mesh, case.params)
+    assert eng.initial_dt(torch.from_numpy(q).cuda(), 0.5) == eng.initial_dt(q, 0.5)
+    q[0, 1, m - 1] = -1.0                # a negative pressure: NaN speeds are passed over
+    assert eng.initial_dt(torch.from_numpy(q).cuda(), 0.5) == eng.initial_dt(q, 0.5)
+    eng.close()
