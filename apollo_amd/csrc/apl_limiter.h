@@ -181,13 +181,21 @@ __global__ void __launch_bounds__(64) lim_average_kernel(LimArgs a) {
   }
 }
 
+// Threads of a workgroup of the gradient pass.  One wave, which a mesh spreads over four times the CUs that
+// groups of 256 reach (us per call, 256 / 64 threads: N = 1, K = 15842 30.5 /
+// 29.0; N = 4, K = 1800 32.9 / 31.1; N = 1, K = 524288 120.3 / 118.9; N = 2, K =
+// 131072 72.3 / 69.7).  Groups of 256 at N > 1 once their rows no longer stay in
+// the caches, since a group's elements are neighbours (K = 320000, a generator's
+// order, 4 variables: N = 2 126 / 129, N = 3 159 / 163, N = 4 160 / 166).
+template <int N>
+static int lim_gradient_threads(int K) {
+  return N > 1 && K >= 262144 ? 256 : 64;
+}
+
 // Two waves per SIMD: at three, which the registers (162) allow, more rows are
 // in flight than the L2 holds (K = 524288, N = 4: 263 -> 266 us per call).
-// One wave per workgroup, which a mesh spreads over four times the CUs that
-// groups of 256 reach (us per call, 256 / 64 threads: N = 1, K = 15842 30.5 /
-// 29.0; N = 4, K = 1800 32.9 / 31.1; N = 1, K = 524288 120.3 / 118.9).
 template <int N, int EQN>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
     lim_gradient_kernel(LimArgs a) {
   static_assert(N <= 4, "the reference's face-end reads leave its face array for N > 4");
   // at N = 1 each XCD takes one contiguous range of elements, so that most

@@ -73,6 +73,17 @@ def test_limiter_periodic_matches_oracle():
     _close(_engine_limit(c, q), want)
 
 
+@pytest.mark.parametrize("N,n", [(2, 362), (2, 363)])
+def test_limiter_large_mesh_matches_oracle(N, n):
+    """K = 262088 and 263538: on either side of the gradient pass's larger
+    workgroups, the last one of the second mesh partial."""
+    case = euler_case(n=n, N=N, m=4)
+    c = Case(case.mesh, E.Params(N, E.EQN_EULER4, limiter=(1.4, 1e-2, 1e-2)), "periodic")
+    q = case.state(amp=5e-2)
+    want = from_oracle(c.params.eqn, O.limit(c.omesh, c.ophys, to_oracle(c.params.eqn, q)))
+    _close(_engine_limit(c, q), want)
+
+
 def test_limit_needs_a_limiter_handle():
     case = ffs_case(N=1, limiter=False)
     eng = E.Engine(case.mesh, case.params)
