@@ -162,8 +162,8 @@ static int dev_alloc(apl_handle *h, void **dst, size_t bytes) {
 
 // The cubature form in FP32 at N <= 3 runs on the VALU kernel unless
 // APL_ALGO_CUBATURE_MFMA asks for the MFMA kernel: measured faster on the 2D
-// Euler vortex at N = 3 (us per fused stage, VALU vs MFMA): K = 8192 15.4 vs
-// 16.8; K = 131072 67.7 vs 75.2.  In FP64 it runs on the even-odd kernel where
+// Euler vortex at N = 3 (us per fused stage, VALU vs MFMA): K = 8192 12.8 vs
+// 15.7; K = 131072 61.9 vs 74.9.  In FP64 it runs on the even-odd kernel where
 // eo_order() says so.
 constexpr bool VALU_BY_DEFAULT = true;
 // The nodal form of MAXWELL_TM3 runs on the VALU kernel under
